@@ -53,12 +53,12 @@ bool ranges_overlap(const void* a, size_t an, const void* b, size_t bn) {
     return a0 < b1 && b0 < a1;
 }
 
-size_t matrix_elems(uint32_t n, uint32_t num_buckets) {
-    if (num_buckets <= 1 || n == 0) return 0;
+// Words of the three-stage path's matrices.
+static size_t stage_matrix_elems(uint32_t n, uint32_t num_buckets) {
     if (num_buckets > 256) {
         // 64-bit elements, and 32-bit ones above kSinglePassBuckets, take
         // passes of at most 256 buckets; 32-bit ones up to it take one pass.
-        size_t m = matrix_elems(n, 256);
+        size_t m = stage_matrix_elems(n, 256);
         if (num_buckets <= kSinglePassBuckets) {
             const int lb = ceil_log2_u32(num_buckets);
             const uint32_t tko = std::min(tile_keys(lb, false, 0), tile_keys(lb, false, kLongTileMin));
@@ -81,6 +81,16 @@ size_t matrix_elems(uint32_t n, uint32_t num_buckets) {
                              ? ((size_t)n + wms_subproblem_keys() - 1) / wms_subproblem_keys()
                              : 0;
     return ((size_t)1 << lb) * std::max(std::max(std::max(t_ko, t_kv), t_w), t_wms);
+}
+
+size_t matrix_elems(uint32_t n, uint32_t num_buckets) {
+    if (num_buckets <= 1 || n == 0) return 0;
+    // Short calls, and the passes of short calls with more buckets, have shorter tiles.
+    size_t m = std::max(stage_matrix_elems(n, num_buckets),
+                        short_matrix_words(n, std::min<uint32_t>(num_buckets, 256u)));
+    if (num_buckets > 256 && num_buckets <= kSinglePassBuckets)
+        m = std::max(m, short_matrix_words(n, num_buckets));
+    return m;
 }
 
 gms_status scratch_alloc(Scratch& s, size_t hist_elems) {
@@ -263,18 +273,30 @@ gms_status run_prescan_only(Scratch& s, const uint32_t* kin, uint32_t n, uint32_
     return hip_status(with_functor(B, d, [&](auto f) { return launch_prescan(c, f); }));
 }
 
-// prescan -> scan -> postscan with the identifier that `with_f` hands to its
-// callback (the built-in kinds by descriptor, or a given functor).
+// The multisplit: one or two launches for short inputs (identifier `any`),
+// else prescan -> scan -> postscan with the identifier that `with_f` hands to
+// its callback (the built-in kinds by descriptor, or a given functor).
 template <class WithF>
 static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
                              uint32_t* vout, uint32_t n, uint32_t B, uint32_t* d_offsets,
-                             hipStream_t stream, Profiler* prof, WithF&& with_f) {
+                             hipStream_t stream, Profiler* prof, const DigitOfF& any,
+                             WithF&& with_f) {
     const bool kv = vin != nullptr;
     if (n == 0) return d_offsets ? hip_status(launch_fill(d_offsets, 0u, B, stream)) : GMS_SUCCESS;
     if (B == 1) {
         hipError_t e = launch_copy(kin, kout, n, stream);
         if (e == hipSuccess && kv) e = launch_copy(vin, vout, n, stream);
         if (e == hipSuccess && d_offsets) e = launch_fill(d_offsets, 0u, 1u, stream);
+        return hip_status(e);
+    }
+    const uint32_t bits = (uint32_t)ceil_log2_u32(B);
+    const bool block = short_one_block(n, bits, 1, kv);
+    const ShortPlan sp = short_plan(n, B, 1, kv);
+    if (block || (sp.items && sp.matrix_words <= s.hist_cap)) {
+        hipEvent_t* ev = (prof && prof->on) ? prof->next(stream) : nullptr;
+        const ShortCall c{kin, vin, kout, vout, n, 1u, kv ? 1u : 0u, d_offsets, B, stream, ev};
+        hipError_t e = block ? launch_short_block(c, bits, any) : launch_short_two(c, sp, s.hist, any);
+        if (e == hipSuccess && ev) e = hipEventRecord(ev[3], stream);
         return hip_status(e);
     }
     MsCall c;
@@ -298,13 +320,14 @@ gms_status run_multisplit(Scratch& s, const uint32_t* kin, const uint32_t* vin, 
                           uint32_t* vout, uint32_t n, uint32_t B, gms_bucket_desc d,
                           uint32_t* d_offsets, hipStream_t stream, Profiler* prof) {
     return run_stages(s, kin, vin, kout, vout, n, B, d_offsets, stream, prof,
+                      DigitOfF{AnyF::make(d.kind, d.param, d.width, B), 0u, ~0u},
                       [&](auto&& launch) { return with_functor(B, d, launch); });
 }
 
 gms_status run_multisplit_digit(Scratch& s, const uint32_t* kin, const uint32_t* vin,
                                 uint32_t* kout, uint32_t* vout, uint32_t n, uint32_t B,
                                 const DigitOfF& f, hipStream_t stream) {
-    return run_stages(s, kin, vin, kout, vout, n, B, nullptr, stream, nullptr,
+    return run_stages(s, kin, vin, kout, vout, n, B, nullptr, stream, nullptr, f,
                       [&](auto&& launch) { return launch(f); });
 }
 
@@ -953,6 +976,11 @@ gms_status gms_sort(gms_sort_ctx* ctx, const uint32_t* kin, uint32_t* kout, cons
                 ranges_overlap(vin, bytes, kout, bytes) || ranges_overlap(kout, bytes, vout, bytes))))
         return GMS_ERR_ALIAS;
     hipStream_t s = (hipStream_t)stream;
+    if (short_one_block(n, 32u, 1, kv)) {  // the whole key is the id
+        const DigitOfF whole{AnyF{0u, ~0u, 0u, 0u, ~0u, ~0u}, 0u, ~0u};
+        const ShortCall c{kin, vin, kout, vout, n, 1u, kv ? 1u : 0u, nullptr, 0u, s};
+        return hip_status(launch_short_block(c, 32u, whole));
+    }
     const uint32_t* sk = kin;
     const uint32_t* sv = vin;
     for (int i = 0; i < np; ++i) {

@@ -192,6 +192,30 @@ struct DigitOf64F {
     GMS_HD uint32_t operator()(uint64_t k) const { return (base(k) >> shift) & mask; }
 };
 
+// The 64-bit range, digit and low-bits identifiers, and digits of their ids,
+// without AnyF64's 64 x 64-bit product (a third of the instructions):
+//   id = floor(k * m / 2^64) | ((k >> shift) & mask), then (id >> shift2) & mask2
+// range: m = B, mask = 0; digit and low bits: m = 0.  Ids are below B by
+// construction (the descriptor check bounds the digit's width).
+struct Lite64F {
+    uint32_t m, shift, mask, shift2, mask2;
+    static constexpr bool covers(uint32_t kind) { return kind == 0 || kind == 2 || kind == 4; }
+    static Lite64F make(uint32_t kind, uint64_t param, uint32_t width, uint32_t num_buckets,
+                        uint32_t shift2, uint32_t mask2) {
+        if (kind == 0) return Lite64F{num_buckets, 0u, 0u, shift2, mask2};
+        if (kind == 2)
+            return Lite64F{0u, (uint32_t)param, width ? (1u << width) - 1u : num_buckets - 1u,
+                           shift2, mask2};
+        return Lite64F{0u, 0u, (1u << (uint32_t)param) - 1u, shift2, mask2};
+    }
+    GMS_HD uint32_t operator()(uint64_t k) const {
+        const uint64_t lo = (uint64_t)(uint32_t)k * m;
+        const uint64_t hi = (uint64_t)(uint32_t)(k >> 32) * m + (lo >> 32);
+        const uint32_t id = (uint32_t)(hi >> 32) | ((uint32_t)(k >> shift) & mask);
+        return (id >> shift2) & mask2;
+    }
+};
+
 // One digit of another identifier's bucket id: (base(k) >> shift) & mask,
 // with base's clamp applied first.  The LSD passes of a multisplit into more
 // than 256 buckets rank by these digits of the (up to 20-bit) bucket id.

@@ -181,6 +181,42 @@ gms_status run_wms_multisplit(Scratch& s, const uint32_t* kin, const uint32_t* v
                               gms_bucket_desc d, uint32_t* d_offsets, bool direct,
                               hipStream_t stream);
 
+// Short inputs (gms_short.hip): one launch on one workgroup, or two launches
+// (a count kernel and a scatter kernel that sums the count matrix itself).
+struct ShortCall {
+    const uint32_t* kin;
+    const uint32_t* vin;  // NULL without values
+    uint32_t* kout;
+    uint32_t* vout;
+    uint32_t n;
+    uint32_t kw, vw;  // words per key and per value
+    uint32_t* offs;   // nb bucket starts (device) or NULL
+    uint32_t nb;
+    hipStream_t stream;
+    hipEvent_t* ev = nullptr;  // stage events (prescan, scan, postscan), if profiled
+};
+// Whether a call of n elements into 2^bits ids fits one workgroup.
+bool short_one_block(uint32_t n, uint32_t bits, uint32_t kw, uint32_t vw);
+// The one-workgroup form; bits <= 32, or 64 for launch_short_sort64 (64-bit keys as ids).
+// Bucket starts are written by the kernel up to kShortBlockOffsets buckets.
+constexpr uint32_t kShortBlockOffsets = 4096;
+hipError_t launch_short_block(const ShortCall& c, uint32_t bits, const DigitOfF& f);
+hipError_t launch_short_block(const ShortCall& c, uint32_t bits, const DigitOf64F& f);
+hipError_t launch_short_block(const ShortCall& c, uint32_t bits, const Lite64F& f);
+hipError_t launch_short_sort64(const ShortCall& c);
+// The two-launch form for ids below num_buckets: its tile and matrix, or
+// items == 0 where the call is not short.
+struct ShortPlan {
+    uint32_t items, group, log_b;
+    size_t matrix_words;
+};
+ShortPlan short_plan(uint32_t n, uint32_t num_buckets, uint32_t kw, uint32_t vw);
+// Matrix words that suffice for the two-launch form of every n up to n_capacity.
+size_t short_matrix_words(uint32_t n_capacity, uint32_t num_buckets);
+hipError_t launch_short_two(const ShortCall& c, const ShortPlan& p, uint32_t* H, const DigitOfF& f);
+hipError_t launch_short_two(const ShortCall& c, const ShortPlan& p, uint32_t* H, const DigitOf64F& f);
+hipError_t launch_short_two(const ShortCall& c, const ShortPlan& p, uint32_t* H, const Lite64F& f);
+
 gms_status hip_status(hipError_t e);
 bool ranges_overlap(const void* a, size_t an, const void* b, size_t bn);
 

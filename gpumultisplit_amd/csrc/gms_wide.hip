@@ -32,11 +32,25 @@ uint32_t wide_min_tile_elems() {
     return m;
 }
 
-template <class Mk64, class Mk32>
+// Calls fn with the identifier of 64-bit keys for one digit (id >> shift) &
+// mask of the descriptor's bucket id (shift 0, mask ~0: the id itself).
+template <class Fn>
+static auto with_id64(const gms_bucket_desc64& d, uint32_t B, uint32_t shift, uint32_t mask, Fn&& fn) {
+    if (Lite64F::covers(d.kind)) return fn(Lite64F::make(d.kind, d.param, d.width, B, shift, mask));
+    return fn(DigitOf64F{AnyF64::make(d.kind, d.param, d.width, B), shift, mask});
+}
+// The same for 32-bit keys.
+static DigitOfF id32(const gms_bucket_desc64& d, uint32_t B, uint32_t shift, uint32_t mask) {
+    return DigitOfF{AnyF::make(d.kind, (uint32_t)d.param, d.width, B), shift, mask};
+}
+
+// One pass into B buckets by the digit (id >> shift) & mask of the ids of
+// descriptor d for `ids` buckets.
 static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* vin,
                               uint32_t* kout, uint32_t* vout, uint32_t n, uint32_t kw,
-                              uint32_t vw, uint32_t B, const Mk64& mk64, const Mk32& mk32,
-                              uint32_t* d_offsets, hipStream_t stream) {
+                              uint32_t vw, uint32_t B, const gms_bucket_desc64& d, uint32_t ids,
+                              uint32_t shift, uint32_t mask, uint32_t* d_offsets,
+                              hipStream_t stream) {
     if (n == 0) return d_offsets ? hip_status(launch_fill(d_offsets, 0u, B, stream)) : GMS_SUCCESS;
     if (B == 1) {
         hipError_t e = launch_copy(kin, kout, (size_t)n * kw, stream);
@@ -45,6 +59,16 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
         return hip_status(e);
     }
     const int lb = ceil_log2_u32(B);
+    // Short inputs: one or two launches.
+    const bool block = short_one_block(n, (uint32_t)lb, kw, vw);
+    const ShortPlan sp = short_plan(n, B, kw, vw);
+    if (block || (sp.items && sp.matrix_words <= s.hist_cap)) {
+        const ShortCall c{kin, vin, kout, vout, n, kw, vw, d_offsets, B, stream};
+        auto go = [&](const auto& f) {
+            return block ? launch_short_block(c, (uint32_t)lb, f) : launch_short_two(c, sp, s.hist, f);
+        };
+        return hip_status(kw == 2 ? with_id64(d, ids, shift, mask, go) : go(id32(d, ids, shift, mask)));
+    }
     const uint32_t tile = wide_tile_elems(kw, vw);
     const uint32_t nt = (uint32_t)(((size_t)n + tile - 1) / tile);
     const size_t m = ((size_t)1 << lb) * nt;
@@ -58,11 +82,20 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
         c.scan_status = s.status;
         c.scan_chunks = scan_chunks(m);
     }
-    hipError_t e = wide_dispatch(c, lb, kw, vw, mk64, mk32, true);
+    auto stage = [&](bool prescan) {
+        if (kw == 2) {
+            const AnyF64 f = AnyF64::make(d.kind, d.param, d.width, ids);
+            return mask == ~0u ? wide_dispatch64(c, lb, vw, f, prescan)
+                               : wide_dispatch64(c, lb, vw, DigitOf64F{f, shift, mask}, prescan);
+        }
+        if (vw != 2) return hipErrorInvalidValue;
+        return wide_stage<1, 2>(c, lb, id32(d, ids, shift, mask), prescan);
+    };
+    hipError_t e = stage(true);
     if (e == hipSuccess)
         e = one ? launch_scan_single(s.hist, s.hist, (uint32_t)m, s.status, stream)
                 : launch_exclusive_scan(s.hist, s.hist, (uint32_t)m, s.part, stream);
-    if (e == hipSuccess) e = wide_dispatch(c, lb, kw, vw, mk64, mk32, false);
+    if (e == hipSuccess) e = stage(false);
     if (e == hipSuccess && d_offsets) e = launch_gather_offsets(s.hist, nt, B, d_offsets, stream);
     return hip_status(e);
 }
@@ -71,10 +104,18 @@ gms_status run_wide_multisplit(Scratch& s, const uint32_t* kin, const uint32_t* 
                                uint32_t* kout, uint32_t* vout, uint32_t n, uint32_t kw,
                                uint32_t vw, uint32_t B, const gms_bucket_desc64& d,
                                uint32_t* d_offsets, hipStream_t stream) {
-    return wide_stages(
-        s, kin, vin, kout, vout, n, kw, vw, B,
-        [&] { return AnyF64::make(d.kind, d.param, d.width, B); },
-        [&] { return AnyF::make(d.kind, (uint32_t)d.param, d.width, B); }, d_offsets, stream);
+    return wide_stages(s, kin, vin, kout, vout, n, kw, vw, B, d, B, 0u, ~0u, d_offsets, stream);
+}
+
+// Bucket starts read off a finished output.
+static gms_status wide_starts(const uint32_t* kout, uint32_t n, uint32_t kw, uint32_t B,
+                              const gms_bucket_desc64& d, uint32_t* d_offsets, hipStream_t stream) {
+    if (kw == 2)
+        return hip_status(launch_bucket_starts<2>(kout, n, B, AnyF64::make(d.kind, d.param, d.width, B),
+                                                  d_offsets, stream));
+    return hip_status(launch_bucket_starts<1>(kout, n, B,
+                                              AnyF::make(d.kind, (uint32_t)d.param, d.width, B),
+                                              d_offsets, stream));
 }
 
 gms_status run_wide_large(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint32_t* kin,
@@ -83,6 +124,14 @@ gms_status run_wide_large(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint
                           uint32_t* d_offsets, hipStream_t stream) {
     if (n == 0) return d_offsets ? hip_status(launch_fill(d_offsets, 0u, B, stream)) : GMS_SUCCESS;
     const int bits = ceil_log2_u32(B);
+    if (short_one_block(n, (uint32_t)bits, kw, vw)) {
+        uint32_t* offs = B <= kShortBlockOffsets ? d_offsets : nullptr;
+        const ShortCall c{kin, vin, kout, vout, n, kw, vw, offs, B, stream};
+        auto go = [&](const auto& f) { return launch_short_block(c, (uint32_t)bits, f); };
+        const hipError_t e = kw == 2 ? with_id64(d, B, 0u, ~0u, go) : go(id32(d, B, 0u, ~0u));
+        if (e != hipSuccess || !d_offsets || offs) return hip_status(e);
+        return wide_starts(kout, n, kw, B, d, d_offsets, stream);
+    }
     const int passes = (bits + 7) / 8;
     const uint32_t* sk = kin;
     const uint32_t* sv = vin;
@@ -93,22 +142,13 @@ gms_status run_wide_large(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint
         uint32_t* dk = to_out ? kout : ktmp;
         uint32_t* dv = vw ? (to_out ? vout : vtmp) : nullptr;
         const uint32_t mask = (1u << w) - 1u;
-        gms_status st = wide_stages(
-            s, sk, sv, dk, dv, n, kw, vw, 1u << w,
-            [&] { return DigitOf64F{AnyF64::make(d.kind, d.param, d.width, B), shift, mask}; },
-            [&] { return DigitOfF{AnyF::make(d.kind, (uint32_t)d.param, d.width, B), shift, mask}; },
-            nullptr, stream);
+        gms_status st = wide_stages(s, sk, sv, dk, dv, n, kw, vw, 1u << w, d, B, shift, mask,
+                                    nullptr, stream);
         if (st != GMS_SUCCESS) return st;
         sk = dk;
         sv = dv;
     }
-    if (!d_offsets) return GMS_SUCCESS;
-    if (kw == 2)
-        return hip_status(launch_bucket_starts<2>(kout, n, B, AnyF64::make(d.kind, d.param, d.width, B),
-                                                  d_offsets, stream));
-    return hip_status(launch_bucket_starts<1>(kout, n, B,
-                                              AnyF::make(d.kind, (uint32_t)d.param, d.width, B),
-                                              d_offsets, stream));
+    return d_offsets ? wide_starts(kout, n, kw, B, d, d_offsets, stream) : GMS_SUCCESS;
 }
 
 int wide_sort_passes(uint32_t key_words, uint32_t digit_bits, SortPass* p) {
@@ -126,6 +166,11 @@ gms_status run_wide_sort(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint3
     SortPass p[16];
     const int np = wide_sort_passes(kw, digit_bits, p);
     if (np == 0) return GMS_ERR_INVALID_ARG;
+    if (short_one_block(n, 32u * kw, kw, vw)) {  // the whole key is the id
+        const ShortCall c{kin, vin, kout, vout, n, kw, vw, nullptr, 0u, stream};
+        return hip_status(kw == 2 ? launch_short_sort64(c)
+                                  : launch_short_block(c, 32u, DigitOfF{AnyF{0u, ~0u, 0u, 0u, ~0u, ~0u}, 0u, ~0u}));
+    }
     const uint32_t* sk = kin;
     const uint32_t* sv = vin;
     for (int i = 0; i < np; ++i) {

@@ -309,22 +309,16 @@ inline hipError_t wide_stage(const WideCall& c, int log_b, const F& f, bool pres
     }
 }
 
-// Stage launch for the element shape; mk64 / mk32 build the identifier of a
-// 64-bit / 32-bit key (only the one the shape uses is built).
-template <class Mk64, class Mk32>
-inline hipError_t wide_dispatch(const WideCall& c, int log_b, uint32_t kw, uint32_t vw,
-                                const Mk64& mk64, const Mk32& mk32, bool prescan) {
-    if (kw == 2) {
-        const auto f = mk64();
-        switch (vw) {
-            case 0: return wide_stage<2, 0>(c, log_b, f, prescan);
-            case 1: return wide_stage<2, 1>(c, log_b, f, prescan);
-            case 2: return wide_stage<2, 2>(c, log_b, f, prescan);
-            default: return hipErrorInvalidValue;
-        }
+// Stage launch for 64-bit keys and vw value words.
+template <class F>
+inline hipError_t wide_dispatch64(const WideCall& c, int log_b, uint32_t vw, const F& f,
+                                  bool prescan) {
+    switch (vw) {
+        case 0: return wide_stage<2, 0>(c, log_b, f, prescan);
+        case 1: return wide_stage<2, 1>(c, log_b, f, prescan);
+        case 2: return wide_stage<2, 2>(c, log_b, f, prescan);
+        default: return hipErrorInvalidValue;
     }
-    if (vw != 2) return hipErrorInvalidValue;
-    return wide_stage<1, 2>(c, log_b, mk32(), prescan);
 }
 
 }  // namespace gms
