@@ -79,8 +79,16 @@ struct Scratch {
     uint32_t* offs = nullptr;  // 256 bucket starts (staging for host offsets)
     uint64_t* status = nullptr;  // single-pass scan statuses of the plain path
     size_t status_cap = 0;       // 64-bit words
+    // Pinned host words that the kernels write the bucket starts of a call with
+    // host results into (pinned_results).
+    uint32_t* pin = nullptr;
     int device = -1;
 };
+// Bucket counts up to which host results go through Scratch::pin.
+constexpr uint32_t kPinnedResults = 1024;
+// s.pin, a slot of the device's pinned block that the first call which needs it
+// takes and scratch_free gives back; NULL when none can be had.
+uint32_t* pinned_results(Scratch& s);
 
 // Multisplits into more than 256 buckets run as a stable radix sort of the
 // bucket ids (gms_large.hip); up to this many buckets.

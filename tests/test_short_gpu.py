@@ -121,3 +121,23 @@ def test_short_sort(dev, kb, vb, bits):
         assert torch.equal(kout, kin[torch.from_numpy(order).to(dev)])
         if vb:
             np.testing.assert_array_equal(vout.cpu().numpy(), order)
+
+
+@pytest.mark.parametrize("B", [2, 1024])
+def test_host_results_of_many_contexts(dev, B):
+    """More contexts alive than pinned result slots: the calls beyond them take
+    the copy, and slots given back are taken again."""
+    n = 5000
+    keys = W.uniform_keys(n, seed=B)
+    wk, _, wo = oracle.multisplit(keys, B, oracle.RANGE, 0, None)
+    kin, kout = to_dev(keys, dev), filled_u32(n, dev)
+    for _ in range(2):
+        ctxs = [gms.multisplit_context(B) for _ in range(67)]
+        for c in ctxs:
+            gms.multisplit_allocate_key_only(n, c)
+            offs = np.full(B, 0xFFFFFFFF, dtype=np.uint32)
+            gms.multisplit_key_only(kin, kout, n, c, gms.range_bucket(B), offs)
+            np.testing.assert_array_equal(offs, wo)
+        np.testing.assert_array_equal(from_dev(kout)[:n], wk)
+        for c in ctxs:
+            gms.multisplit_release_memory(c)
