@@ -263,6 +263,12 @@ __device__ __forceinline__ void store_device_u32(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #endif
 }
+// Waits for every outstanding memory operation of the wave.
+__device__ __forceinline__ void wait_loads() {
+#ifndef GMS_HOST_EMULATION
+    __builtin_amdgcn_s_waitcnt(0);
+#endif
+}
 // Short pause in a wait loop.
 __device__ __forceinline__ void wait_pause() {
 #ifndef GMS_HOST_EMULATION

@@ -4,8 +4,8 @@
 // A resident grid (two workgroups per CU) walks full tiles of 256 x 16 words
 // with unconditional 16-byte loads, issuing the next tile's loads before it
 // counts the current one, so every workgroup keeps a tile in flight while its
-// waves add bins into their own LDS sub-histograms (ds_add).  The ragged tail
-// (< one tile) is counted by workgroup 0 with guarded loads.  Each workgroup
+// waves add bins into the workgroup's LDS histograms (ds_add).  The ragged ends
+// (< one tile) are counted by the last workgroup with guarded loads.  Each workgroup
 // folds its sub-histograms and adds its non-zero bins to the global
 // histogram once at the end.
 #include "gms_internal.hpp"
@@ -16,9 +16,9 @@ namespace gms {
 constexpr int kHistItems = 16;
 constexpr uint32_t kHistTile = kThreads * kHistItems;
 constexpr uint32_t kHistGrid = 512;
-constexpr uint32_t kRangeGrid = 1024;
-constexpr int kHistCopies = 8;
-constexpr int kRangeCopies = 4;
+constexpr uint32_t kRangeGrid = 768;
+constexpr int kHistCopies = 32;
+constexpr int kRangeCopies = 16;
 
 // bins_of(x, b) maps a register array of words to bins (>= nbins: not
 // counted); it sees a whole tile row at once so that a kernel can issue the
@@ -27,50 +27,72 @@ constexpr int kRangeCopies = 4;
 // elements, and bins_of reports an element's bin at its first word and an
 // out-of-range bin at its others.  n counts elements.
 //
-// Every wave counts into C copies of its sub-histogram, lane l into copy
-// l % C, with rows of 257 words so that the copies of one bin lie in
-// different banks.  Keys that share a bin across a wave (sorted runs, one
-// dominant bin) then add to C addresses instead of one, which the LDS
-// serialises per address; evenly spread keys see the same bank spread as
-// with one copy.
-template <bool VEC, int W = 1, int C = kHistCopies, bool STREAM = false, class BinsOf>
-__device__ __forceinline__ void hist_body(const uint32_t* __restrict__ p, uint32_t n, uint32_t nbins,
-                                          uint32_t* __restrict__ d_hist, BinsOf bins_of) {
+// The workgroup counts into C copies of its histogram, thread t into copy
+// t % C, with rows of 257 words so that the copies of one bin lie in different
+// banks.  Keys that share a bin across a wave (sorted runs, one dominant bin)
+// then add to C addresses instead of one, which the LDS serialises per address;
+// evenly spread keys see the same bank spread as with one copy.  Word 256 of a
+// row is never read: bins_of may send what is not counted there.
+//
+// The up to three words before the first 16-byte boundary and the ragged tail
+// are counted by the last workgroup, so inputs that start off a boundary (a slice of a
+// larger array) take the vector loads too.
+template <int W = 1, int C = kHistCopies, bool STREAM = false, class BinsOf>
+__device__ __forceinline__ void hist_body(const uint32_t* __restrict__ words, uint32_t num,
+                                          uint32_t nbins, uint32_t* __restrict__ d_hist,
+                                          BinsOf bins_of) {
     static_assert(W == 1 || W == 2, "elements of 1 or 2 words");
     static_assert(C >= 1 && C <= 64 && (C & (C - 1)) == 0, "copies: a power of two");
-    constexpr uint32_t ROW = C > 1 ? 257u : 256u;
-    constexpr uint32_t NH = (uint32_t)(kWaves * C);
+    constexpr uint32_t ROW = 257u;
+    constexpr uint32_t NH = (uint32_t)C;
     __shared__ uint32_t s_h[NH * ROW];
-    const uint32_t tid = threadIdx.x, wid = tid >> 6;
+    const uint32_t tid = threadIdx.x;
     for (uint32_t i = tid; i < NH * ROW; i += kThreads) s_h[i] = 0;
     __syncthreads();
-    uint32_t* my = s_h + (wid * (uint32_t)C + (tid & (uint32_t)(C - 1))) * ROW;
+    uint32_t* my = s_h + (tid & (NH - 1u)) * ROW;
+    const uint32_t to16 = (uint32_t)((0u - (uint32_t)((uintptr_t)words >> 2)) & 3u) / W;
+    const uint32_t head = to16 < num ? to16 : num;
+    const uint32_t* p = words + (size_t)head * W;
+    const uint32_t n = num - head;
     const uint32_t nfull = (uint32_t)((size_t)n * W / kHistTile);
     uint32_t t = blockIdx.x;
     uint32_t x[kHistItems];
-    if (t < nfull) load_striped4_full<kHistItems, VEC, STREAM>(p, (size_t)t * kHistTile, x);
+    if (t < nfull) load_striped4_full<kHistItems, true, STREAM>(p, (size_t)t * kHistTile, x);
+    // The first tile arrives before the loop: with it possibly pending at the
+    // loop's head, the compiler waits there, in every iteration, for the loads
+    // that the iteration has just issued, and nothing is prefetched.
+    wait_loads();
     while (t < nfull) {
         const uint32_t tn = t + gridDim.x;
         uint32_t y[kHistItems];
-        if (tn < nfull) load_striped4_full<kHistItems, VEC, STREAM>(p, (size_t)tn * kHistTile, y);
+        if (tn < nfull) load_striped4_full<kHistItems, true, STREAM>(p, (size_t)tn * kHistTile, y);
         uint32_t b[kHistItems];
         bins_of(x, b);
 #pragma unroll
         for (int k = 0; k < kHistItems; ++k)
-            if (b[k] < nbins) atomicAdd(&my[b[k]], 1u);
+            if (b[k] <= 256u) atomicAdd(&my[b[k]], 1u);
 #pragma unroll
         for (int k = 0; k < kHistItems; ++k) x[k] = y[k];
         t = tn;
     }
-    if (blockIdx.x == 0) {
-        for (size_t e = (size_t)nfull * (kHistTile / W) + tid; e < n; e += kThreads) {
-            uint32_t xt[W], bt[W];
+    if (blockIdx.x == gridDim.x - 1u) {
+        // As a tile with guarded loads (a second one for at most three elements).
+        constexpr uint32_t STEP = kHistTile / W;
+        const uint32_t tail = n - nfull * STEP, rest = head + tail;
+        for (uint32_t i0 = 0; i0 < rest; i0 += STEP) {
 #pragma unroll
-            for (int w = 0; w < W; ++w) xt[w] = p[e * W + w];
-            bins_of(xt, bt);
+            for (int k = 0; k < kHistItems; k += W) {
+                const uint32_t i = i0 + (uint32_t)(k / W) * kThreads + tid;
+                const size_t e = i < head ? i : (size_t)num - tail + (i - head);
 #pragma unroll
-            for (int w = 0; w < W; ++w)
-                if (bt[w] < nbins) atomicAdd(&my[bt[w]], 1u);
+                for (int w = 0; w < W; ++w) x[k + w] = i < rest ? words[e * W + w] : 0u;
+            }
+            uint32_t b[kHistItems];
+            bins_of(x, b);
+#pragma unroll
+            for (int k = 0; k < kHistItems; ++k)
+                if (i0 + (uint32_t)(k / W) * kThreads + tid < rest && b[k] <= 256u)
+                    atomicAdd(&my[b[k]], 1u);
         }
     }
     __syncthreads();
@@ -94,20 +116,20 @@ __device__ __forceinline__ auto per_word(F f) {
 
 // STREAM: streamed loads, for inputs of at least kStreamLoadMin words (each
 // line is read once and the input is larger than the caches).
-template <bool VEC, bool STREAM, class F>
+template <bool STREAM, class F>
 __global__ __launch_bounds__(kThreads) void hist_u32_kernel(const uint32_t* __restrict__ kin,
                                                             uint32_t n, uint32_t nbins,
                                                             uint32_t* __restrict__ d_hist, F f) {
-    hist_body<VEC, 1, kHistCopies, STREAM>(kin, n, nbins, d_hist,
+    hist_body<1, kHistCopies, STREAM>(kin, n, nbins, d_hist,
                                            per_word([&](uint32_t k) { return f(k); }));
 }
 
-template <bool VEC, bool STREAM>
+template <bool STREAM>
 __global__ __launch_bounds__(kThreads) void hist_even_f32_kernel(const uint32_t* __restrict__ xbits,
                                                                  uint32_t n, uint32_t nbins,
                                                                  uint32_t* __restrict__ d_hist,
                                                                  float lower, float inv_delta) {
-    hist_body<VEC, 1, kHistCopies, STREAM>(xbits, n, nbins, d_hist, per_word([&](uint32_t w) {
+    hist_body<1, kHistCopies, STREAM>(xbits, n, nbins, d_hist, per_word([&](uint32_t w) {
         const float d = __uint_as_float(w) - lower;
         // The product is rounded on its own (no contraction with a later add);
         // negative, NaN and >= nbins samples map to an out-of-range bin.
@@ -123,18 +145,23 @@ __global__ __launch_bounds__(kThreads) void hist_even_f32_kernel(const uint32_t*
 //
 // Every workgroup first builds a table over kRangeCells equal cells of
 // [levels[0], levels[nl-1]): cell c holds lo_c = #{interior edges j with
-// cell(levels[j]) < c} and cnt_c = #{j : cell(levels[j]) == c}.  cell() is
-// non-decreasing and the same function is applied to samples and edges, so
-// for a sample x in cell c every edge in a lower cell is < x and every edge in
-// a higher one is > x: its bin lies in [lo_c, lo_c + cnt_c].  Most cells hold
-// no edge and the sample's bin is lo_c after one LDS read; the others finish
-// with a binary search of floor(log2(cnt_c)) + 1 steps over the edges, which
-// are staged in LDS padded with the type's largest value.  The table reads of
-// a thread's 16 samples are issued together, and the search runs the same
-// floor(log2(max_c cnt_c)) + 1 steps for every sample, a sample joining at
-// the first step h <= cnt_c; samples outside it read a broadcast word.
+// cell(levels[j]) < c}, cnt_c = #{j : cell(levels[j]) == c} and, for cnt_c = 1,
+// that edge.  cell() is non-decreasing and the same function is applied to
+// samples and edges, so for a sample x in cell c every edge in a lower cell is
+// < x and every edge in a higher one is > x: its bin lies in [lo_c, lo_c + cnt_c].
+// Two LDS reads and one compare, bin = lo_c + (x >= edge), settle every sample
+// whose cell has at most one edge (an empty cell holds an edge above all
+// samples); the others search the cell's edges in LDS.  With 257 random edges
+// one wave row in nine has such a sample.  A table of lo_c and cnt_c alone,
+// with a search of as many steps as the fullest cell needs for every sample,
+// took 72 us for 2^26 and 136 us for 2^27 samples on MI355X (sorted samples 92 and
+// 167), this one 62 and 108 (56 and 97).
+//
+// Building the table takes a workgroup several microseconds.  Inputs of at most
+// one tile per workgroup do without it (TABLE = false): a branch-free search of
+// eight steps over the edges for every sample.
 constexpr uint32_t kRangeCells = 4096;
-constexpr uint32_t kCellsPerThread = kRangeCells / kThreads;
+static_assert(kRangeCells == 16u * kThreads, "16 cells per thread");
 
 template <class T>
 struct RangeCellF;
@@ -170,88 +197,128 @@ struct RangeCellF<uint32_t> {
 };
 static_assert(kRangeCells == (1u << 12), "the integer cell shift assumes 2^12 cells");
 
-template <class T, bool VEC>
+template <class T>
+__device__ __forceinline__ uint32_t bits_of(T v) {
+    uint32_t w;
+    __builtin_memcpy(&w, &v, sizeof w);
+    return w;
+}
+template <class T>
+__device__ __forceinline__ T value_of(uint32_t w) {
+    T v;
+    __builtin_memcpy(&v, &w, sizeof v);
+    return v;
+}
+
+template <class T, bool TABLE, bool STREAM>
 __global__ __launch_bounds__(kThreads) void hist_range_kernel(const uint32_t* __restrict__ xbits,
                                                               uint32_t n, uint32_t nl,
                                                               const T* __restrict__ d_levels,
                                                               uint32_t* __restrict__ d_hist) {
-    __shared__ __attribute__((aligned(16))) uint32_t s_tab[kRangeCells];  // lo_c | cnt_c << 16
-    __shared__ T s_lv[512];
+    constexpr uint32_t CELLS = TABLE ? kRangeCells : 4u;
+    __shared__ __attribute__((aligned(16))) uint32_t s_cell[CELLS];  // lo_c | cnt_c << 16
+    __shared__ __attribute__((aligned(16))) uint32_t s_edge[CELLS];
+    __shared__ T s_lv[256];  // levels[i] for i < nb, then the pad
     __shared__ uint32_t s_ws[kWaves];
-    __shared__ uint32_t s_maxcnt;
-    const uint32_t tid = threadIdx.x, nb = nl - 1u;
+    const uint32_t tid = threadIdx.x, nb = nl - 1u;  // nb <= 256: one edge per thread
     const T lo_edge = d_levels[0], hi_edge = d_levels[nb];
+    const T pad = RangeCellF<T>::pad();
+    const T lv = tid < nb ? d_levels[tid] : pad;
+    s_lv[tid] = lv;
     const RangeCellF<T> cell(lo_edge, hi_edge);
-    // s_lv[i] = levels[i] for i < nb, then the pad (index <= lo_c + 2^steps - 1 <= 510)
-    for (uint32_t i = tid; i < 512u; i += kThreads) s_lv[i] = i < nb ? d_levels[i] : RangeCellF<T>::pad();
-    uint32_t* mine = s_tab + tid * kCellsPerThread;
+    if constexpr (TABLE) {
+        // A thread's 16 cells as four 16-byte vectors, in an order that spreads
+        // the lanes over the banks.
+        uint4* row = reinterpret_cast<uint4*>(s_cell) + 4u * tid;
+        const uint32_t pw = bits_of<T>(pad);
 #pragma unroll
-    for (uint32_t i = 0; i < kCellsPerThread; i += 4)
-        *reinterpret_cast<uint4*>(mine + i) = make_uint4(0u, 0u, 0u, 0u);
-    if (tid == 0) s_maxcnt = 0;
-    __syncthreads();
-    for (uint32_t j = tid + 1u; j < nb; j += kThreads) atomicAdd(&s_tab[cell(d_levels[j])], 1u);
-    __syncthreads();
-    uint32_t c[kCellsPerThread], sum = 0, mx = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < kCellsPerThread; i += 4) {
-        const uint4 v = *reinterpret_cast<const uint4*>(mine + i);
-        c[i] = v.x; c[i + 1] = v.y; c[i + 2] = v.z; c[i + 3] = v.w;
-        sum += v.x + v.y + v.z + v.w;
-        mx = std::max(mx, std::max(std::max(v.x, v.y), std::max(v.z, v.w)));
-    }
-    if (mx) atomicMax(&s_maxcnt, mx);
-    uint32_t total;
-    uint32_t run = block_excl_scan<kWaves>(sum, s_ws, total);  // its barrier also orders s_maxcnt
-    const uint32_t maxcnt = GMS_READFIRSTLANE(s_maxcnt);
-    const uint32_t h0 = maxcnt ? 1u << (31 - __builtin_clz(maxcnt)) : 0u;  // first search step
-#pragma unroll
-    for (uint32_t i = 0; i < kCellsPerThread; ++i) {
-        const uint32_t e = run | (c[i] << 16);
-        run += c[i];
-        c[i] = e;
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < kCellsPerThread; i += 4)
-        *reinterpret_cast<uint4*>(mine + i) = make_uint4(c[i], c[i + 1], c[i + 2], c[i + 3]);
-    // (hist_body's first barrier orders the table before any lookup)
-    // Four sub-histogram copies per wave (35 KB of LDS per workgroup with the
-    // cell table: the grid of kRangeGrid = 4 workgroups per CU is resident):
-    // sorted samples, whose lanes share a bin, contend on 4 addresses instead
-    // of one.
-    hist_body<VEC, 1, kRangeCopies>(xbits, n, nb, d_hist, [&](auto& x, auto& b) {
-        constexpr int N = (int)(sizeof(x) / sizeof(x[0]));
-        T v[N];
-        uint32_t cnt[N];
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            __builtin_memcpy(&v[k], &x[k], sizeof(T));
-            const uint32_t e = s_tab[cell(v[k])];  // any word maps to a cell
-            b[k] = e & 0xFFFFu;
-            cnt[k] = e >> 16;
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t r = (i + (tid >> 2)) & 3u;
+            row[r] = make_uint4(0u, 0u, 0u, 0u);
+            reinterpret_cast<uint4*>(s_edge)[4u * tid + r] = make_uint4(pw, pw, pw, pw);
         }
-        for (uint32_t h = h0; h; h >>= 1) {
+        __syncthreads();
+        const bool interior = tid > 0u && tid < nb;
+        const uint32_t mine = interior ? cell(lv) : 0u;
+        if (interior) atomicAdd(&s_cell[mine], 1u);
+        __syncthreads();
+        // Sums of the vectors in cell order, then their exclusive prefixes.
+        uint4 v[4];
+        uint32_t part[4], sum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t r = (i + (tid >> 2)) & 3u;
+            v[i] = row[r];
+            const uint32_t q = v[i].x + v[i].y + v[i].z + v[i].w;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) part[j] = j == r ? q : part[j];
+            sum += q;
+        }
+        uint32_t total;
+        const uint32_t run = block_excl_scan<kWaves>(sum, s_ws, total);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t r = (i + (tid >> 2)) & 3u;
+            uint32_t a = run;
+#pragma unroll
+            for (uint32_t j = 0; j < 3; ++j) a += j < r ? part[j] : 0u;
+            const uint32_t b = a + v[i].x, c = b + v[i].y, d = c + v[i].z;
+            row[r] = make_uint4(a | (v[i].x << 16), b | (v[i].y << 16), c | (v[i].z << 16),
+                                d | (v[i].w << 16));
+        }
+        __syncthreads();
+        if (interior && s_cell[mine] >> 16 == 1u) s_edge[mine] = bits_of<T>(lv);
+    }
+    // (hist_body's first barrier orders the table and the levels before any lookup)
+    hist_body<1, kRangeCopies, STREAM>(xbits, n, nb, d_hist, [&](auto& x, auto& b) {
+        constexpr int N = (int)(sizeof(x) / sizeof(x[0]));
+        if constexpr (TABLE) {
+            uint32_t e[N], g[N];
 #pragma unroll
             for (int k = 0; k < N; ++k) {
-                // inactive samples add 0 whatever they read
-                const uint32_t hk = h <= cnt[k] ? h : 0u;
-                const uint32_t idx = hk ? b[k] + hk : 0u;
-                b[k] += v[k] >= s_lv[idx] ? hk : 0u;
+                const uint32_t c = cell(value_of<T>(x[k]));  // any word maps to a cell
+                e[k] = s_cell[c];
+                g[k] = s_edge[c];
+            }
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const T v = value_of<T>(x[k]);
+                const uint32_t cnt = e[k] >> 16, lo = e[k] & 0xFFFFu;
+                b[k] = lo + (v >= value_of<T>(g[k]) ? 1u : 0u);
+                if (cnt > 1u) {  // the number of the cell's edges that are <= v
+                    uint32_t l = 0, h = cnt;
+                    while (l < h) {
+                        const uint32_t m = (l + h) >> 1;
+                        if (v >= s_lv[lo + 1u + m]) l = m + 1u;
+                        else h = m;
+                    }
+                    b[k] = lo + l;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < N; ++k) b[k] = 0;
+#pragma unroll
+            for (uint32_t h = 128; h; h >>= 1) {
+#pragma unroll
+                for (int k = 0; k < N; ++k) b[k] += value_of<T>(x[k]) >= s_lv[b[k] + h] ? h : 0u;
             }
         }
 #pragma unroll
-        for (int k = 0; k < N; ++k)
-            if (!(v[k] >= lo_edge && v[k] < hi_edge)) b[k] = 0xFFFFFFFFu;  // outside, or NaN
+        for (int k = 0; k < N; ++k) {
+            const T v = value_of<T>(x[k]);
+            if (!(v >= lo_edge && v < hi_edge)) b[k] = 256u;  // outside, or NaN: not counted
+        }
     });
 }
 
 // 64-bit keys through a 64-bit identifier: the same prefetching resident
 // grid over the key array viewed as words, each (low, high) word pair one key.
-template <bool VEC, bool STREAM>
+template <bool STREAM>
 __global__ __launch_bounds__(kThreads) void hist_u64_kernel(const uint32_t* __restrict__ words,
                                                             uint32_t n, uint32_t nbins,
                                                             uint32_t* __restrict__ d_hist, AnyF64 f) {
-    hist_body<VEC, 2, kHistCopies, STREAM>(words, n, nbins, d_hist, [&](auto& x, auto& b) {
+    hist_body<2, kHistCopies, STREAM>(words, n, nbins, d_hist, [&](auto& x, auto& b) {
         constexpr int N = (int)(sizeof(x) / sizeof(x[0]));
 #pragma unroll
         for (int k = 0; k < N; k += 2) {
@@ -261,43 +328,36 @@ __global__ __launch_bounds__(kThreads) void hist_u64_kernel(const uint32_t* __re
     });
 }
 
-static uint32_t hist_grid(uint32_t n, uint32_t max_grid = kHistGrid) {
-    const uint32_t full = n / kHistTile;
-    return full < max_grid ? (full ? full : 1u) : max_grid;
+// A workgroup per full tile and one for the ragged ends, up to the resident grid.
+static uint32_t hist_grid(uint32_t n, uint32_t max_grid = kHistGrid, uint32_t words = 1) {
+    const size_t grid = (size_t)n * words / kHistTile + 1;
+    return grid < max_grid ? (uint32_t)grid : max_grid;
 }
 
-static bool aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
 static bool stream_words(size_t words) { return words >= kStreamLoadMin; }
 
 hipError_t launch_histogram_u64(const uint64_t* keys, uint32_t n, uint32_t* d_hist,
                                 uint32_t nbins, const AnyF64& f, hipStream_t stream) {
-    const size_t full = (size_t)n * 2 / kHistTile;
-    const uint32_t grid = full < kHistGrid ? (full ? (uint32_t)full : 1u) : kHistGrid;
+    const uint32_t grid = hist_grid(n, kHistGrid, 2);
     const uint32_t* w = reinterpret_cast<const uint32_t*>(keys);
-    if (aligned16(keys) && stream_words((size_t)n * 2))
-        hipLaunchKernelGGL((hist_u64_kernel<true, true>), dim3(grid), dim3(kThreads), 0, stream,
-                           w, n, nbins, d_hist, f);
-    else if (aligned16(keys))
-        hipLaunchKernelGGL((hist_u64_kernel<true, false>), dim3(grid), dim3(kThreads), 0, stream,
-                           w, n, nbins, d_hist, f);
+    if (stream_words((size_t)n * 2))
+        hipLaunchKernelGGL((hist_u64_kernel<true>), dim3(grid), dim3(kThreads), 0, stream, w, n,
+                           nbins, d_hist, f);
     else
-        hipLaunchKernelGGL((hist_u64_kernel<false, false>), dim3(grid), dim3(kThreads), 0, stream,
-                           w, n, nbins, d_hist, f);
+        hipLaunchKernelGGL((hist_u64_kernel<false>), dim3(grid), dim3(kThreads), 0, stream, w, n,
+                           nbins, d_hist, f);
     return hipGetLastError();
 }
 
 template <class F>
 static hipError_t launch_hist(const uint32_t* kin, uint32_t n, uint32_t* d_hist, uint32_t nbins,
                               const F& f, hipStream_t stream) {
-    if (aligned16(kin) && stream_words(n))
-        hipLaunchKernelGGL((hist_u32_kernel<true, true, F>), dim3(hist_grid(n)), dim3(kThreads),
-                           0, stream, kin, n, nbins, d_hist, f);
-    else if (aligned16(kin))
-        hipLaunchKernelGGL((hist_u32_kernel<true, false, F>), dim3(hist_grid(n)), dim3(kThreads),
-                           0, stream, kin, n, nbins, d_hist, f);
+    if (stream_words(n))
+        hipLaunchKernelGGL((hist_u32_kernel<true, F>), dim3(hist_grid(n)), dim3(kThreads), 0,
+                           stream, kin, n, nbins, d_hist, f);
     else
-        hipLaunchKernelGGL((hist_u32_kernel<false, false, F>), dim3(hist_grid(n)), dim3(kThreads),
-                           0, stream, kin, n, nbins, d_hist, f);
+        hipLaunchKernelGGL((hist_u32_kernel<false, F>), dim3(hist_grid(n)), dim3(kThreads), 0,
+                           stream, kin, n, nbins, d_hist, f);
     return hipGetLastError();
 }
 
@@ -322,12 +382,16 @@ static hipError_t launch_range(const void* x, uint32_t n, int32_t* d_hist, uint3
                                const T* d_levels, hipStream_t stream) {
     const uint32_t* xb = reinterpret_cast<const uint32_t*>(x);
     uint32_t* h = reinterpret_cast<uint32_t*>(d_hist);
-    if (aligned16(x))
-        hipLaunchKernelGGL((hist_range_kernel<T, true>), dim3(hist_grid(n, kRangeGrid)),
-                           dim3(kThreads), 0, stream, xb, n, num_levels, d_levels, h);
+    const dim3 grid(hist_grid(n, kRangeGrid)), block(kThreads);
+    if (n / kHistTile < kRangeGrid)
+        hipLaunchKernelGGL((hist_range_kernel<T, false, false>), grid, block, 0, stream, xb, n,
+                           num_levels, d_levels, h);
+    else if (!stream_words(n))
+        hipLaunchKernelGGL((hist_range_kernel<T, true, false>), grid, block, 0, stream, xb, n,
+                           num_levels, d_levels, h);
     else
-        hipLaunchKernelGGL((hist_range_kernel<T, false>), dim3(hist_grid(n, kRangeGrid)),
-                           dim3(kThreads), 0, stream, xb, n, num_levels, d_levels, h);
+        hipLaunchKernelGGL((hist_range_kernel<T, true, true>), grid, block, 0, stream, xb, n,
+                           num_levels, d_levels, h);
     return hipGetLastError();
 }
 
@@ -347,15 +411,12 @@ hipError_t launch_histogram_even_f32(const float* x, uint32_t n, int32_t* d_hist
                                      float lower, float inv_delta, hipStream_t stream) {
     const uint32_t* xb = reinterpret_cast<const uint32_t*>(x);
     uint32_t* h = reinterpret_cast<uint32_t*>(d_hist);
-    if (aligned16(x) && stream_words(n))
-        hipLaunchKernelGGL((hist_even_f32_kernel<true, true>), dim3(hist_grid(n)), dim3(kThreads),
-                           0, stream, xb, n, nbins, h, lower, inv_delta);
-    else if (aligned16(x))
-        hipLaunchKernelGGL((hist_even_f32_kernel<true, false>), dim3(hist_grid(n)),
-                           dim3(kThreads), 0, stream, xb, n, nbins, h, lower, inv_delta);
+    if (stream_words(n))
+        hipLaunchKernelGGL((hist_even_f32_kernel<true>), dim3(hist_grid(n)), dim3(kThreads), 0,
+                           stream, xb, n, nbins, h, lower, inv_delta);
     else
-        hipLaunchKernelGGL((hist_even_f32_kernel<false, false>), dim3(hist_grid(n)),
-                           dim3(kThreads), 0, stream, xb, n, nbins, h, lower, inv_delta);
+        hipLaunchKernelGGL((hist_even_f32_kernel<false>), dim3(hist_grid(n)), dim3(kThreads), 0,
+                           stream, xb, n, nbins, h, lower, inv_delta);
     return hipGetLastError();
 }
 
