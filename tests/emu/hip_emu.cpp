@@ -1,11 +1,15 @@
 // Workgroup execution for the host emulation (see hip_emu.hpp).
 #include "hip_emu.hpp"
 
-#include <condition_variable>
+#include <ucontext.h>
+
 #include <memory>
 #include <mutex>
-#include <thread>
 #include <vector>
+
+#ifdef __SANITIZE_ADDRESS__
+#include <sanitizer/common_interface_defs.h>
+#endif
 
 namespace gms_emu {
 
@@ -13,15 +17,74 @@ thread_local gms_emu_dim3 thread_idx = {0, 0, 0};
 gms_emu_dim3 block_idx = {0, 0, 0}, block_dim = {1, 1, 1}, grid_dim = {1, 1, 1};
 
 namespace {
-std::unique_ptr<std::barrier<>> g_block_barrier;
-std::vector<std::unique_ptr<std::barrier<>>> g_wave_barrier;
+// The threads of a workgroup are fibers of the launching host thread.  A
+// fiber runs until it meets a wave or workgroup barrier; the scheduler in
+// launch() lets it go on when every live fiber of its wave (workgroup) waits
+// at one.  (One host thread per GPU thread spent nearly all its time in
+// futex calls.)
+enum class State { ready, at_wave, at_block, done };
+constexpr size_t kStack = 96 * 1024;
+struct Fiber {
+    ucontext_t ctx;
+    std::unique_ptr<char[]> stack;
+    State state = State::done;
+    void* fake = nullptr;
+};
+std::vector<std::unique_ptr<Fiber>> g_fibers;
+ucontext_t g_sched;
+void* g_sched_fake = nullptr;
+const void* g_sched_bottom = nullptr;
+size_t g_sched_size = 0;
+std::function<void()>* g_body = nullptr;
+uint32_t g_current = 0;
 uint32_t g_wave_buf[1024];
 std::mutex g_launch_mutex;
+
+#ifdef __SANITIZE_ADDRESS__
+void leave(void** fake, const void* bottom, size_t size) {
+    __sanitizer_start_switch_fiber(fake, bottom, size);
+}
+void arrive(void* fake, const void** bottom, size_t* size) {
+    __sanitizer_finish_switch_fiber(fake, bottom, size);
+}
+#else
+void leave(void**, const void*, size_t) {}
+void arrive(void*, const void**, size_t*) {}
+#endif
+
+void fiber_main() {
+    arrive(nullptr, &g_sched_bottom, &g_sched_size);
+    (*g_body)();
+    Fiber& f = *g_fibers[g_current];
+    f.state = State::done;
+    leave(nullptr, g_sched_bottom, g_sched_size);  // never comes back
+    swapcontext(&f.ctx, &g_sched);
+}
+
+void run_fiber(uint32_t i) {
+    Fiber& f = *g_fibers[i];
+    g_current = i;
+    thread_idx = {i, 0, 0};
+    leave(&g_sched_fake, f.stack.get(), kStack);
+    swapcontext(&g_sched, &f.ctx);
+    arrive(g_sched_fake, nullptr, nullptr);
+}
+
+void wait_at(State s) {
+    Fiber& f = *g_fibers[g_current];
+    f.state = s;
+    leave(&f.fake, g_sched_bottom, g_sched_size);
+    swapcontext(&f.ctx, &g_sched);
+    arrive(f.fake, &g_sched_bottom, &g_sched_size);
+}
 }  // namespace
 
-void syncthreads() { g_block_barrier->arrive_and_wait(); }
+void syncthreads() { wait_at(State::at_block); }
 
-static std::barrier<>& wave_barrier() { return *g_wave_barrier[thread_idx.x >> 6]; }
+struct WaveBarrier {
+    void arrive_and_wait() { wait_at(State::at_wave); }
+};
+static WaveBarrier wave_barrier() { return {}; }
 
 uint32_t update_dpp(uint32_t old, uint32_t src, int ctrl, int row_mask, int bank_mask,
                     bool bound_ctrl) {
@@ -85,21 +148,48 @@ void launch(dim3 grid, dim3 block, std::function<void()> body) {
     }
     grid_dim = {grid.x, 1, 1};
     block_dim = {nt, 1, 1};
-    g_block_barrier = std::make_unique<std::barrier<>>((std::ptrdiff_t)nt);
-    g_wave_barrier.clear();
-    for (uint32_t w = 0; w < (nt + 63) / 64; ++w)
-        g_wave_barrier.push_back(std::make_unique<std::barrier<>>((std::ptrdiff_t)(nt < 64 ? nt : 64)));
+    while (g_fibers.size() < nt) {
+        g_fibers.push_back(std::make_unique<Fiber>());
+        g_fibers.back()->stack.reset(new char[kStack]);
+    }
+    g_body = &body;
     for (uint32_t b = 0; b < grid.x; ++b) {
         block_idx = {b, 0, 0};
-        std::vector<std::thread> th;
-        th.reserve(nt);
-        for (uint32_t t = 0; t < nt; ++t)
-            th.emplace_back([t, &body]() {
-                thread_idx = {t, 0, 0};
-                body();
-            });
-        for (auto& x : th) x.join();
+        for (uint32_t t = 0; t < nt; ++t) {
+            Fiber& f = *g_fibers[t];
+            getcontext(&f.ctx);
+            f.ctx.uc_stack.ss_sp = f.stack.get();
+            f.ctx.uc_stack.ss_size = kStack;
+            f.ctx.uc_link = nullptr;
+            makecontext(&f.ctx, fiber_main, 0);
+            f.state = State::ready;
+        }
+        for (bool live = true; live;) {
+            live = false;
+            for (uint32_t w = 0; w < nt; w += 64) {  // every wave up to its workgroup barrier
+                const uint32_t end = w + 64 < nt ? w + 64 : nt;
+                for (bool again = true; again;) {
+                    uint32_t at_wave = 0, at_block = 0;
+                    for (uint32_t t = w; t < end; ++t) {
+                        if (g_fibers[t]->state == State::ready) run_fiber(t);
+                        at_wave += g_fibers[t]->state == State::at_wave;
+                        at_block += g_fibers[t]->state == State::at_block;
+                    }
+                    if (at_wave && at_block) {
+                        fprintf(stderr, "hip_emu: a wave waits at two different barriers\n");
+                        abort();
+                    }
+                    again = at_wave != 0;
+                    live = live || at_block != 0;
+                    for (uint32_t t = w; t < end && again; ++t)
+                        if (g_fibers[t]->state == State::at_wave) g_fibers[t]->state = State::ready;
+                }
+            }
+            for (uint32_t t = 0; t < nt; ++t)
+                if (g_fibers[t]->state == State::at_block) g_fibers[t]->state = State::ready;
+        }
     }
+    thread_idx = {0, 0, 0};
 }
 
 std::atomic<uint64_t> alloc_calls{0};

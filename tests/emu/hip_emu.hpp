@@ -4,8 +4,8 @@
 // tests of the real kernel code at small sizes).
 //
 // Execution model: a kernel launch runs its workgroups one after another;
-// every workgroup is blockDim.x host threads that meet at __syncthreads()
-// (a std::barrier).  __shared__ arrays become function-static storage, which
+// every workgroup is blockDim.x fibers that meet at __syncthreads().
+// __shared__ arrays become function-static storage, which
 // is what LDS is to a sequence of workgroups.  DPP lane moves and readlane
 // are wave collectives: the 64 threads of a wave publish their values and
 // meet at a wave barrier.  All kernel call sites of these collectives are in
@@ -17,7 +17,6 @@
 #include <string.h>
 
 #include <atomic>
-#include <barrier>
 #include <chrono>
 #include <cstdio>
 #include <functional>
