@@ -119,10 +119,23 @@ gms_status BatchEngine::reserve_tables(uint32_t instances, uint64_t work_items) 
     return GMS_SUCCESS;
 }
 
+// Tile shape of a step that was not tuned.  Steps of few keys are bound by the
+// latency of a tile and by their ragged tiles, large ones by bandwidth, where
+// longer output runs pay.  On MI355X (us a run at 8 / 16 / 24 keys per thread):
+// 64 buckets 1.1M pairs 17 / 23 / 25, 11M 48 / 56 / 62, 72M 355 / 303 / 301; 256
+// buckets 11M 61 / 64 / 66; sorts and multisplits of 36M pairs 361 / 344 / 359.
+static uint32_t default_items(const gms_batch_item* items, uint32_t count) {
+    uint64_t keys = 0;
+    for (uint32_t i = 0; i < count; ++i) keys += items[i].n;
+    return keys < (1u << 24) ? 8u : keys < (1u << 26) ? 16u : 24u;
+}
+
 gms_status BatchEngine::plan(const gms_batch_item* items, uint32_t count,
                              const BatchWideItem* wide, uint32_t wcount, int slot) {
-    const uint32_t K = tuning.items_per_thread;
+    const uint32_t K = tuning.items_per_thread ? tuning.items_per_thread
+                                               : default_items(items, count);
     if (K != 8 && K != 16 && K != 24 && K != 32) return GMS_ERR_INVALID_ARG;
+    items_ = K;
     const uint32_t tile = (uint32_t)kThreads * K;
     slot_ = slot & 1;
     PinnedVec<BatchInst>& hi = h_inst_[slot_];
@@ -248,7 +261,8 @@ size_t BatchEngine::device_bytes() const {
     return align256(std::max<size_t>(num_instances, 1) * sizeof(BatchInst)) +
            align256(std::max<size_t>(num_wide, 1) * sizeof(BatchWideInst)) +
            align256(std::max<size_t>(num_work, 1) * sizeof(BatchWork)) + align256(m * 4) +
-           align256(scan_partials_needed(m) * 4) + align256(16 * std::max<size_t>(groups.size(), 1) * 4);
+           align256(scan_partials_needed(m) * 4) + align256(scan_chunks(m) * sizeof(uint64_t)) +
+           align256(16 * std::max<size_t>(groups.size(), 1) * 4);
 }
 
 BatchDevice BatchEngine::carve(void* base) const {
@@ -265,6 +279,8 @@ BatchDevice BatchEngine::carve(void* base) const {
     p += align256(m * 4);
     d.part = (uint32_t*)p;
     p += align256(scan_partials_needed(m) * 4);
+    d.status = (uint64_t*)p;
+    p += align256(scan_chunks(m) * sizeof(uint64_t));
     d.queue = (uint32_t*)p;
     return d;
 }
@@ -296,7 +312,7 @@ uint32_t BatchEngine::grid_for(const BatchGroup& g, bool post) const {
     const uint32_t nw = g.w1 - g.w0;
     if (!tuning.persistent) return nw;
     int occ = 1;
-    switch (tuning.items_per_thread) {
+    switch (items_) {
         case 8: occ = batch_occupancy_k8(g.log_b, g.kv, post); break;
         case 16: occ = batch_occupancy_k16(g.log_b, g.kv, post); break;
         case 24: occ = batch_occupancy_k24(g.log_b, g.kv, post); break;
@@ -311,19 +327,26 @@ uint32_t BatchEngine::grid_for(const BatchGroup& g, bool post) const {
 uint32_t BatchEngine::launches() const {
     if (num_work == 0) return 0;
     return (tuning.persistent && !groups.empty() ? 1u : 0u) +
-           2u * (uint32_t)(groups.size() + wide_groups.size()) + (m_total ? 3u : 0u);
+           2u * (uint32_t)(groups.size() + wide_groups.size()) + (m_total ? 3u : 0u);  // the scan: at most three
 }
 
 gms_status BatchEngine::launch(const BatchDevice& d, hipStream_t s) {
     if (num_work == 0) return GMS_SUCCESS;
     const uint32_t G = (uint32_t)groups.size();
     hipError_t e = tuning.persistent && G ? launch_fill(d.queue, 0u, 16 * G, s) : hipSuccess;
+    // The one-launch scan up to kScanFusedParts chunks (every chunk adds the
+    // totals of all chunks before it); its status words are cleared by the
+    // step's first prescan.
+    const uint32_t chunks = scan_chunks(m_total);
+    uint32_t nclear = chunks <= kScanFusedParts ? chunks : 0u;
+    const bool single = nclear != 0;
     auto one = [&](const BatchGroup& g, uint32_t gi, bool post) {
         BatchLaunch c{d.inst, d.work + g.w0, g.w1 - g.w0, grid_for(g, post), d.mat,
                       (uint32_t)m_total, (uint32_t)keys_total, d.queue + 16 * gi + (post ? 8 : 0),
                       g.log_b, g.kv, g.vec, tuning.persistent != 0, s,
-                      keys_total >= kStreamLoadMin};
-        switch (tuning.items_per_thread) {
+                      keys_total >= kStreamLoadMin, d.status, post ? 0u : nclear};
+        nclear = 0;
+        switch (items_) {
             case 8: return post ? launch_batch_postscan_k8(c) : launch_batch_prescan_k8(c);
             case 16: return post ? launch_batch_postscan_k16(c) : launch_batch_prescan_k16(c);
             case 24: return post ? launch_batch_postscan_k24(c) : launch_batch_prescan_k24(c);
@@ -332,14 +355,17 @@ gms_status BatchEngine::launch(const BatchDevice& d, hipStream_t s) {
     };
     auto wide_one = [&](const BatchWideGroup& g, bool post) {
         const BatchWideLaunch c{d.winst, d.work + g.w0, g.w1 - g.w0, d.mat, (uint32_t)m_total,
-                                (uint32_t)keys_total, g.log_b, g.kw, g.vw, g.vec, s};
+                                (uint32_t)keys_total, g.log_b, g.kw, g.vw, g.vec, s,
+                                d.status, post ? 0u : nclear};
+        nclear = 0;
         return launch_batch_wide(c, post);
     };
     for (uint32_t gi = 0; gi < G && e == hipSuccess; ++gi) e = one(groups[gi], gi, false);
     for (size_t gi = 0; gi < wide_groups.size() && e == hipSuccess; ++gi)
         e = wide_one(wide_groups[gi], false);
     if (e == hipSuccess)
-        e = launch_exclusive_scan(d.mat, d.mat, (uint32_t)m_total, d.part, s);
+        e = single ? launch_scan_single(d.mat, d.mat, (uint32_t)m_total, d.status, s)
+                   : launch_exclusive_scan(d.mat, d.mat, (uint32_t)m_total, d.part, s);
     for (uint32_t gi = 0; gi < G && e == hipSuccess; ++gi) e = one(groups[gi], gi, true);
     for (size_t gi = 0; gi < wide_groups.size() && e == hipSuccess; ++gi)
         e = wide_one(wide_groups[gi], true);
@@ -655,7 +681,10 @@ gms_status gms_batch_set_tuning(gms_batch* b, gms_batch_tuning t) {
 
 gms_status gms_batch_get_tuning(const gms_batch* b, gms_batch_tuning* t) {
     if (!b || !t) return GMS_ERR_INVALID_ARG;
-    t->items_per_thread = b->tuning.items_per_thread;
+    // not tuned: the shape the first step was planned with
+    t->items_per_thread = b->tuning.items_per_thread ? b->tuning.items_per_thread
+                          : b->eng.empty()           ? 24u
+                                                     : b->eng[0]->items_per_thread();
     t->persistent = b->tuning.persistent;
     return GMS_SUCCESS;
 }

@@ -63,7 +63,7 @@ struct BatchWideGroup {
 };
 
 struct BatchTuning {
-    uint32_t items_per_thread = 24;  // 8, 16, 24 or 32 keys per thread (tile = 256 x this)
+    uint32_t items_per_thread = 0;   // 8, 16, 24 or 32 keys per thread (tile = 256 x this); 0: by size
     uint32_t persistent = 0;         // 0: one workgroup per tile; 1: resident grid + work queue
 };
 
@@ -74,6 +74,7 @@ struct BatchDevice {
     BatchWork* work = nullptr;
     uint32_t* mat = nullptr;    // concatenated histogram matrix
     uint32_t* part = nullptr;   // scan partials
+    uint64_t* status = nullptr; // status words of the single-pass scan
     uint32_t* queue = nullptr;  // 8 per-XCD work-queue counters per launch
 };
 
@@ -109,8 +110,10 @@ class BatchEngine {
     std::vector<BatchGroup> groups;
     std::vector<BatchWideGroup> wide_groups;
     uint32_t launches() const;
+    uint32_t items_per_thread() const { return items_; }  // of the current plan
 
   private:
+    uint32_t items_ = 24;
     int slot_ = 0;
     PinnedVec<BatchInst> h_inst_[2];
     PinnedVec<BatchWideInst> h_winst_[2];

@@ -15,6 +15,7 @@
 #pragma once
 
 #include "gms_kernels.hpp"
+#include "gms_rank.hpp"
 
 namespace gms {
 
@@ -68,6 +69,8 @@ struct BatchWideLaunch {
     uint32_t kw, vw;
     bool vec;
     hipStream_t stream;
+    uint64_t* clear = nullptr;  // scan status words the prescan clears
+    uint32_t nclear = 0;
 };
 hipError_t launch_batch_wide(const BatchWideLaunch& c, bool post);
 
@@ -121,11 +124,16 @@ __device__ __forceinline__ void batch_prescan_item(const BatchInst* __restrict__
 }
 
 // STREAM: streamed key loads, for batches larger than the caches (whose
-// postscans cannot find the keys still cached).
+// postscans cannot find the keys still cached).  `clear` (nclear 64-bit words):
+// the status words of the step's single-pass scan, zeroed by workgroup 0 of the
+// step's first prescan.
 template <int LOG_B, int K, bool VEC, bool PERSIST, bool STREAM = false>
 __global__ __launch_bounds__(kThreads) void ms_batch_prescan_kernel(
     const BatchInst* __restrict__ inst, const BatchWork* __restrict__ work, uint32_t num_work,
-    uint32_t* __restrict__ H, uint32_t* __restrict__ queue) {
+    uint32_t* __restrict__ H, uint32_t* __restrict__ queue, uint64_t* __restrict__ clear,
+    uint32_t nclear) {
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < nclear; i += kThreads) store_device_u64(&clear[i], 0ull);
     constexpr int B = 1 << LOG_B;
     __shared__ __attribute__((aligned(16))) uint32_t s_h[kWaves * B];
     if constexpr (!PERSIST) {
@@ -139,8 +147,11 @@ __global__ __launch_bounds__(kThreads) void ms_batch_prescan_kernel(
     }
 }
 
+// Tiles of 32 keys per thread rank with LDS counters (postscan_rank): register
+// counters would leave one workgroup per CU (11M pairs into 64 buckets 91 to
+// 115 us, against 82).
 template <int LOG_B, int K, int LEVEL_BITS, bool KV, bool VEC, bool ALIAS>
-__device__ __forceinline__ void batch_postscan_item(
+__device__ __forceinline__ void batch_postscan_item_lds(
     const BatchInst* __restrict__ inst, const BatchWork* __restrict__ work, uint32_t w,
     const uint32_t* __restrict__ G, uint32_t m_total, uint32_t keys_total, uint32_t* s_keys,
     uint32_t* s_vals, uint32_t* s_cnt, uint32_t* s_delta, uint32_t* s_bs, uint32_t* s_ws) {
@@ -188,40 +199,110 @@ __device__ __forceinline__ void batch_postscan_item(
     }
 }
 
-template <int LOG_B, int K, int LEVEL_BITS, bool KV, bool VEC, bool PERSIST>
+// LDS of the batched postscan.
+template <int LOG_B, int K, bool KV>
+struct BatchSmem {
+    static constexpr uint32_t TILE = kThreads * K;
+    static constexpr int W = rank_pass_bits(LOG_B);
+    uint32_t keys[TILE];
+    uint32_t vals[KV ? TILE : 4];
+    uint32_t cnt[rank_cnt_words<W, kThreads>()];
+    uint32_t ws[rank_ws_words<W, kThreads>()];
+    uint32_t delta[1 << LOG_B];
+    uint32_t bs[kWaves];
+};
+
+// Ranked with register counters (gms_rank.hpp), as the short-input kernels: a
+// step's tiles are mostly few and ragged, and what bounds them is the latency
+// of one tile.
+template <int LOG_B, int K, bool KV, bool VEC>
+__device__ __forceinline__ void batch_postscan_item(const BatchInst* __restrict__ inst,
+                                                    const BatchWork* __restrict__ work, uint32_t w,
+                                                    const uint32_t* __restrict__ G,
+                                                    uint32_t m_total, uint32_t keys_total,
+                                                    BatchSmem<LOG_B, K, KV>& sm) {
+    constexpr int B = 1 << LOG_B;
+    constexpr uint32_t TILE = kThreads * K;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
+    const BatchWork it = work[w];
+    const BatchInst& I = inst[it.inst];
+    const uint32_t t = it.tile;
+    const uint32_t nvalid = tile_valid(I.n, t, TILE);
+    const size_t base = (size_t)t * TILE;
+
+    uint32_t key[K], val[K];
+    load_words<K>(I.kin + base, tid * (uint32_t)K, nvalid, VEC, key);
+    if constexpr (KV) load_words<K>(I.vin + base, tid * (uint32_t)K, nvalid, VEC, val);
+    else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) val[k] = 0;
+    }
+
+    // G[b][t] of this instance and the next word in scan order; the word
+    // after the whole concatenation is the batch's key total.
+    const uint32_t bt = tid < (uint32_t)B ? tid : (uint32_t)B - 1u;
+    const uint32_t idx = I.mbase + bt * I.num_tiles + t;
+    const uint32_t g0 = G[idx];
+    const uint32_t g1 = idx + 1u < m_total ? G[idx + 1u] : keys_total;
+    const uint32_t cnt = tid < (uint32_t)B ? g1 - g0 : 0u;
+    const uint32_t g0l = g0 - I.obase;  // start inside this instance's output
+    if (t == 0 && I.offs && tid < I.nb) I.offs[tid] = g0l;
+    const uint32_t inc = wave_incl_scan(cnt);
+    if (lane == 63u) sm.bs[wid] = inc;
+    auto deltas = [&] {
+        uint32_t ls = inc - cnt;
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)kWaves; ++i) ls += i < wid ? sm.bs[i] : 0u;
+        if (tid < (uint32_t)B) sm.delta[tid] = g0l - ls;
+    };
+    if (nvalid == TILE) {
+        rank_tile<LOG_B, kThreads, K, KV, true>(key, val, TILE, I.f, sm.keys, sm.vals, sm.cnt,
+                                                sm.ws, deltas);
+        postscan_write<K, KV, true>(TILE, I.n, I.kout, I.vout, I.f, sm.keys, sm.vals, sm.delta);
+    } else {
+        rank_tile<LOG_B, kThreads, K, KV, false>(key, val, nvalid, I.f, sm.keys, sm.vals, sm.cnt,
+                                                 sm.ws, deltas);
+        postscan_write<K, KV, false>(nvalid, I.n, I.kout, I.vout, I.f, sm.keys, sm.vals, sm.delta);
+    }
+}
+
+template <int LOG_B, int K, bool KV, bool VEC, bool PERSIST>
 __global__ __launch_bounds__(kThreads) void ms_batch_postscan_kernel(
     const BatchInst* __restrict__ inst, const BatchWork* __restrict__ work, uint32_t num_work,
     const uint32_t* __restrict__ G, uint32_t m_total, uint32_t keys_total,
     uint32_t* __restrict__ queue) {
-    constexpr int B = 1 << LOG_B;
-    constexpr uint32_t TILE = kThreads * K;
-    constexpr int NLEV = (LOG_B + LEVEL_BITS - 1) / LEVEL_BITS;
-    static_assert(NLEV >= 1 && NLEV <= 3, "at most three ranking passes");
-    static_assert(K % 4 == 0, "vector loads");
-
-    constexpr uint32_t CNT = cnt_words(LEVEL_BITS);
-    constexpr bool ALIAS = tune_alias(LOG_B, K, KV, LEVEL_BITS);
-    __shared__ __attribute__((aligned(16))) uint32_t s_keys[TILE];
-    __shared__ __attribute__((aligned(16))) uint32_t s_vc[KV ? TILE : CNT];
-    __shared__ __attribute__((aligned(16))) uint32_t s_cnt_sep[(KV && !ALIAS) ? CNT : 4];
-    __shared__ uint32_t s_delta[B];
-    __shared__ uint32_t s_bs[kWaves];
-    __shared__ uint32_t s_ws[kWaves];
-    uint32_t* s_vals = s_vc;
-    uint32_t* s_cnt = KV ? (ALIAS ? s_vc : s_cnt_sep) : s_vc;
-
-    if constexpr (!PERSIST) {
-        batch_postscan_item<LOG_B, K, LEVEL_BITS, KV, VEC, ALIAS>(
-            inst, work, xcd_tile(blockIdx.x, num_work), G, m_total, keys_total, s_keys, s_vals,
-            s_cnt, s_delta, s_bs, s_ws);
+    auto each = [&](auto&& item) {
+        if constexpr (!PERSIST) {
+            item(xcd_tile(blockIdx.x, num_work));
+        } else {
+            __shared__ uint32_t s_next;
+            const XcdRange R = xcd_range(num_work);
+            for (uint32_t i = blockIdx.x / 8u; i < R.count; i = xcd_next(queue, R.wgs, &s_next))
+                item(R.begin + i);
+        }
+    };
+    if constexpr (K < 32) {
+        __shared__ __attribute__((aligned(16))) BatchSmem<LOG_B, K, KV> sm;
+        each([&](uint32_t w) {
+            batch_postscan_item<LOG_B, K, KV, VEC>(inst, work, w, G, m_total, keys_total, sm);
+        });
     } else {
-        __shared__ uint32_t s_next;
-        const XcdRange R = xcd_range(num_work);
-        for (uint32_t i = blockIdx.x / 8u; i < R.count; i = xcd_next(queue, R.wgs, &s_next))
-            batch_postscan_item<LOG_B, K, LEVEL_BITS, KV, VEC, ALIAS>(inst, work, R.begin + i, G,
-                                                                m_total, keys_total, s_keys,
-                                                                s_vals, s_cnt, s_delta, s_bs,
-                                                                s_ws);
+        constexpr uint32_t TILE = kThreads * K;
+        constexpr int LB = tune_level_bits(LOG_B);
+        constexpr uint32_t CNT = cnt_words(LB);
+        constexpr bool ALIAS = tune_alias(LOG_B, K, KV, LB);
+        __shared__ __attribute__((aligned(16))) uint32_t s_keys[TILE];
+        __shared__ __attribute__((aligned(16))) uint32_t s_vc[KV ? TILE : CNT];
+        __shared__ __attribute__((aligned(16))) uint32_t s_cnt_sep[(KV && !ALIAS) ? CNT : 4];
+        __shared__ uint32_t s_delta[1 << LOG_B];
+        __shared__ uint32_t s_bs[kWaves];
+        __shared__ uint32_t s_ws[kWaves];
+        uint32_t* s_cnt = KV && !ALIAS ? s_cnt_sep : s_vc;
+        each([&](uint32_t w) {
+            batch_postscan_item_lds<LOG_B, K, LB, KV, VEC, ALIAS>(inst, work, w, G, m_total,
+                                                                  keys_total, s_keys, s_vc, s_cnt,
+                                                                  s_delta, s_bs, s_ws);
+        });
     }
 }
 
@@ -241,6 +322,8 @@ struct BatchLaunch {
     bool persistent;
     hipStream_t stream;
     bool stream_loads = false;  // the step is larger than the caches: prescan loads stream
+    uint64_t* clear = nullptr;  // scan status words the prescan clears
+    uint32_t nclear = 0;
 };
 
 hipError_t launch_batch_prescan_k8(const BatchLaunch& c);
@@ -262,7 +345,8 @@ struct BatchKernels {
     template <int LOG_B, bool VEC, bool P, bool S = false>
     static hipError_t prescan_v(const BatchLaunch& c) {
         hipLaunchKernelGGL((ms_batch_prescan_kernel<LOG_B, K, VEC, P, S>), dim3(c.grid),
-                           dim3(kThreads), 0, c.stream, c.inst, c.work, c.num_work, c.H, c.queue);
+                           dim3(kThreads), 0, c.stream, c.inst, c.work, c.num_work, c.H, c.queue, c.clear,
+                           c.nclear);
         return hipGetLastError();
     }
     template <int LOG_B>
@@ -276,8 +360,7 @@ struct BatchKernels {
     }
     template <int LOG_B, bool KV, bool VEC, bool P>
     static hipError_t postscan_v(const BatchLaunch& c) {
-        constexpr int LB = tune_level_bits(LOG_B);
-        hipLaunchKernelGGL((ms_batch_postscan_kernel<LOG_B, K, LB, KV, VEC, P>), dim3(c.grid),
+        hipLaunchKernelGGL((ms_batch_postscan_kernel<LOG_B, K, KV, VEC, P>), dim3(c.grid),
                            dim3(kThreads), 0, c.stream, c.inst, c.work, c.num_work,
                            (const uint32_t*)c.H, c.m_total, c.keys_total, c.queue);
         return hipGetLastError();
@@ -293,9 +376,8 @@ struct BatchKernels {
         int occ = 0;
         hipError_t e;
         if (post) {
-            constexpr int LB = tune_level_bits(LOG_B);
             e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &occ, ms_batch_postscan_kernel<LOG_B, K, LB, KV, true, true>, kThreads, 0);
+                &occ, ms_batch_postscan_kernel<LOG_B, K, KV, true, true>, kThreads, 0);
         } else {
             e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &occ, ms_batch_prescan_kernel<LOG_B, K, true, true>, kThreads, 0);

@@ -11,7 +11,9 @@ namespace gms {
 template <int LOG_B, int KW, int VW, bool VEC>
 __global__ __launch_bounds__(kThreads) void ms_batch_wide_prescan_kernel(
     const BatchWideInst* __restrict__ inst, const BatchWork* __restrict__ work, uint32_t num_work,
-    uint32_t* __restrict__ H) {
+    uint32_t* __restrict__ H, uint64_t* __restrict__ clear, uint32_t nclear) {
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < nclear; i += kThreads) store_device_u64(&clear[i], 0ull);
     constexpr int K = wide_items(KW, VW);
     __shared__ __attribute__((aligned(16))) uint32_t s_h[kWaves * (1 << LOG_B)];
     const BatchWork it = work[xcd_tile(blockIdx.x, num_work)];
@@ -67,10 +69,10 @@ static hipError_t batch_wide_b(const BatchWideLaunch& c, bool post) {
     } else {
         if (c.vec)
             hipLaunchKernelGGL((ms_batch_wide_prescan_kernel<LOG_B, KW, VW, true>), grid, block, 0,
-                               c.stream, c.inst, c.work, c.num_work, c.H);
+                               c.stream, c.inst, c.work, c.num_work, c.H, c.clear, c.nclear);
         else
             hipLaunchKernelGGL((ms_batch_wide_prescan_kernel<LOG_B, KW, VW, false>), grid, block,
-                               0, c.stream, c.inst, c.work, c.num_work, c.H);
+                               0, c.stream, c.inst, c.work, c.num_work, c.H, c.clear, c.nclear);
     }
     return hipGetLastError();
 }

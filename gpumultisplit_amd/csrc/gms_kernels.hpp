@@ -67,6 +67,23 @@ __device__ __forceinline__ void load_blocked_guarded(const uint32_t* __restrict_
     for (int k = 0; k < K; ++k) x[k] = (off + (uint32_t)k < nvalid) ? p[base + off + k] : 0u;
 }
 
+// NW consecutive words from word `off` of p, zero from word `nvalid` on.
+// `vec`: p + off may be read in 16-byte vectors.
+template <int NW>
+__device__ __forceinline__ void load_words(const uint32_t* __restrict__ p, uint32_t off,
+                                           uint32_t nvalid, bool vec, uint32_t (&x)[NW]) {
+    if (NW % 4 == 0 && vec && off + (uint32_t)NW <= nvalid) {
+#pragma unroll
+        for (int i = 0; i < NW / 4; ++i) {
+            const uint4 v = reinterpret_cast<const uint4*>(p + off)[i];
+            x[4 * i + 0] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) x[i] = off + (uint32_t)i < nvalid ? p[off + i] : 0u;
+    }
+}
+
 // Striped by 16 bytes: thread t owns [4(j*256+t), +4) for j < K/4.  Every
 // line is read by one instruction, so the vector loads may stream
 // (STREAM: ld_stream, the line not kept for reuse).  That pays for inputs

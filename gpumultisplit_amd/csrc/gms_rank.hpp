@@ -33,10 +33,11 @@ constexpr uint32_t rank_ws_words() {
     return (uint32_t)(rank_words<W>() * (NT / 64) < 64 ? 64 : rank_words<W>() * (NT / 64));
 }
 
-// Step 1: slot[k] = rank of element k among the thread's earlier elements of
-// its digit; c[j] = count of digit j (low half) and of digit j + DP (high half).
-template <int W, int K>
-__device__ __forceinline__ void rank_count(const uint32_t (&dig)[K], uint32_t (&slot)[K],
+// Step 1: slot[k] = digit of element k << 8 | its rank among the thread's
+// earlier elements of that digit (one register per element until its position
+// is known); c[j] = count of digit j (low half) and of digit j + DP (high half).
+template <int W, int K, class Digit>
+__device__ __forceinline__ void rank_count(Digit digit, uint32_t (&slot)[K],
                                            uint32_t (&c)[rank_words<W>()]) {
     constexpr int DP = rank_words<W>();
     static_assert(W >= 1 && W <= 4, "1 to 4 bits per pass");
@@ -45,8 +46,8 @@ __device__ __forceinline__ void rank_count(const uint32_t (&dig)[K], uint32_t (&
         uint32_t p = 0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            const uint32_t sh = dig[k] * 8u;
-            slot[k] = (p >> sh) & 255u;
+            const uint32_t d = digit(k), sh = d * 8u;
+            slot[k] = ((p >> sh) & 255u) | (d << 8);
             p += 1u << sh;
         }
 #pragma unroll
@@ -56,68 +57,57 @@ __device__ __forceinline__ void rank_count(const uint32_t (&dig)[K], uint32_t (&
         uint64_t p = 0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            const uint32_t sh = dig[k] * 8u;
-            slot[k] = (uint32_t)(p >> sh) & 255u;
+            const uint32_t d = digit(k), sh = d * 8u;
+            slot[k] = ((uint32_t)(p >> sh) & 255u) | (d << 8);
             p += (uint64_t)1 << sh;
         }
         const uint32_t lo = (uint32_t)p, hi = (uint32_t)(p >> 32);
 #pragma unroll
         for (int j = 0; j < DP; ++j)
             c[j] = ((lo >> (8 * j)) & 255u) | (((hi >> (8 * j)) & 255u) << 16);
-    } else if constexpr (K <= 30) {  // sixteen 4-bit counters, for at most 15 elements at a time
-        constexpr int G = K <= 15 ? K : (K + 1) / 2;
-        uint64_t a = 0, b = 0;
+    } else {
+        // Sixteen 4-bit counters, for groups of at most 15 elements; an
+        // element's rank adds the counts of the groups before its own.
+        constexpr int NG = (K + 14) / 15, G = (K + NG - 1) / NG;
+        uint64_t p[NG];
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            const uint32_t sh = dig[k] * 4u;
-            slot[k] = (uint32_t)(a >> sh) & 15u;
-            a += (uint64_t)1 << sh;
-        }
+        for (int g = 0; g < NG; ++g) {
+            p[g] = 0;
 #pragma unroll
-        for (int k = G; k < K; ++k) {
-            const uint32_t sh = dig[k] * 4u;
-            slot[k] = ((uint32_t)(a >> sh) & 15u) + ((uint32_t)(b >> sh) & 15u);
-            b += (uint64_t)1 << sh;
+            for (int k = g * G; k < (g + 1) * G && k < K; ++k) {
+                const uint32_t d = digit(k), sh = d * 4u;
+                uint32_t r = d << 8;
+#pragma unroll
+                for (int q = 0; q <= g; ++q) r += (uint32_t)(p[q] >> sh) & 15u;
+                slot[k] = r;
+                p[g] += (uint64_t)1 << sh;
+            }
         }
-        const uint32_t al = (uint32_t)a, ah = (uint32_t)(a >> 32);
-        const uint32_t bl = (uint32_t)b, bh = (uint32_t)(b >> 32);
 #pragma unroll
         for (int j = 0; j < DP; ++j) {
-            c[j] = ((al >> (4 * j)) & 15u) | (((ah >> (4 * j)) & 15u) << 16);
-            if constexpr (K > G) c[j] += ((bl >> (4 * j)) & 15u) | (((bh >> (4 * j)) & 15u) << 16);
-        }
-    } else {  // sixteen byte counters in two registers pairs
-        uint64_t lo = 0, hi = 0;
+            c[j] = 0;
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const uint32_t sh = (dig[k] & 7u) * 8u;
-            const bool up = (dig[k] & 8u) != 0;
-            const uint64_t p = up ? hi : lo;
-            slot[k] = (uint32_t)(p >> sh) & 255u;
-            const uint64_t q = p + ((uint64_t)1 << sh);
-            hi = up ? q : hi;
-            lo = up ? lo : q;
+            for (int g = 0; g < NG; ++g)
+                c[j] += (((uint32_t)p[g] >> (4 * j)) & 15u) |
+                        ((((uint32_t)(p[g] >> 32) >> (4 * j)) & 15u) << 16);
         }
-#pragma unroll
-        for (int j = 0; j < DP; ++j)
-            c[j] = ((uint32_t)(lo >> (8 * j)) & 255u) | (((uint32_t)(hi >> (8 * j)) & 255u) << 16);
     }
 }
 
-// pos[k] for every element.  `mid` runs after the barrier (work of the caller
+// pos[k] for every element; digit(k) gives its digit.  `mid` runs after the barrier (work of the caller
 // that needs one).  s_cnt: rank_cnt_words words, s_ws: rank_ws_words words;
 // the caller puts a barrier between the use of pos (its scatter) and the next
 // call.
-template <int W, int NT, int K, class Mid>
-__device__ __forceinline__ void rank_digits(const uint32_t (&dig)[K], uint32_t (&pos)[K],
-                                            uint32_t* s_cnt, uint32_t* s_ws, Mid mid) {
+template <int W, int NT, int K, class Digit, class Mid>
+__device__ __forceinline__ void rank_digits(Digit digit, uint32_t (&pos)[K], uint32_t* s_cnt,
+                                            uint32_t* s_ws, Mid mid) {
     constexpr int DP = rank_words<W>();
     constexpr int NW = NT / 64;
     static_assert((uint64_t)NT * K <= 65535u, "16-bit positions");
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wid = (uint32_t)GMS_READFIRSTLANE((int)(tid >> 6));
     uint32_t c[DP], inc[DP];
-    rank_count<W, K>(dig, pos, c);
+    rank_count<W, K>(digit, pos, c);
 #pragma unroll
     for (int j = 0; j < DP; ++j) inc[j] = wave_incl_scan(c[j]);
     if (lane == 63u) {
@@ -162,8 +152,69 @@ __device__ __forceinline__ void rank_digits(const uint32_t (&dig)[K], uint32_t (
     mid();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const uint32_t v = col[(dig[k] & (uint32_t)(DP - 1)) * (uint32_t)NT];
-        pos[k] += (dig[k] & (uint32_t)DP) ? v >> 16 : v & 0xFFFFu;
+        const uint32_t d = pos[k] >> 8;
+        const uint32_t v = col[(d & (uint32_t)(DP - 1)) * (uint32_t)NT];
+        pos[k] = (pos[k] & 255u) + ((d & (uint32_t)DP) ? v >> 16 : v & 0xFFFFu);
+    }
+}
+
+// Bits of the ranking passes of a LOG_B-bit id: one pass up to 4 bits, then
+// 3 + 3 (2), 4 + 4 (3), and 3 or 4 bits in three passes.
+constexpr int rank_pass_bits(int log_b) { return log_b <= 4 ? log_b : (log_b <= 6 || log_b == 9 ? 3 : 4); }
+
+template <int SHIFT, int W, int NT, int K, bool KV, bool FULL, class F, class Mid>
+__device__ __forceinline__ void rank_tile_pass(const uint32_t (&key)[K], const uint32_t (&val)[K],
+                                               uint32_t nvalid, F f, uint32_t* s_keys,
+                                               uint32_t* s_vals, uint32_t* s_cnt, uint32_t* s_ws,
+                                               Mid mid) {
+    constexpr uint32_t DM = (1u << W) - 1u;
+    const uint32_t first = threadIdx.x * (uint32_t)K;
+    uint32_t pos[K];
+    rank_digits<W, NT, K>(
+        [&](int k) { return FULL || first + (uint32_t)k < nvalid ? (f(key[k]) >> SHIFT) & DM : DM; },
+        pos, s_cnt, s_ws, mid);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        s_keys[pos[k]] = key[k];
+        if constexpr (KV) s_vals[pos[k]] = val[k];
+    }
+    __syncthreads();
+}
+
+// Leaves the tile's nvalid keys (and values) in s_keys (s_vals), stably sorted
+// by the LOG_B-bit id f(key); key and val hold the thread's K consecutive keys
+// of the tile.  Keys past nvalid take the largest digit of every pass and stay
+// behind.  `mid` runs after the first pass's barrier; ends with a barrier.
+template <int LOG_B, int NT, int K, bool KV, bool FULL, class F, class Mid>
+__device__ __forceinline__ void rank_tile(uint32_t (&key)[K], uint32_t (&val)[K], uint32_t nvalid,
+                                          F f, uint32_t* s_keys, uint32_t* s_vals,
+                                          uint32_t* s_cnt, uint32_t* s_ws, Mid mid) {
+    constexpr int W = rank_pass_bits(LOG_B);
+    rank_tile_pass<0, W, NT, K, KV, FULL>(key, val, nvalid, f, s_keys, s_vals, s_cnt, s_ws, mid);
+    auto reload = [&] {
+        static_assert(K % 4 == 0, "16-byte LDS reads of whole rows");
+        const uint32_t off = threadIdx.x * (uint32_t)K;
+#pragma unroll
+        for (int i = 0; i < K / 4; ++i) {
+            const uint4 a = *reinterpret_cast<const uint4*>(s_keys + off + 4 * i);
+            key[4 * i + 0] = a.x; key[4 * i + 1] = a.y; key[4 * i + 2] = a.z; key[4 * i + 3] = a.w;
+            if constexpr (KV) {
+                const uint4 b = *reinterpret_cast<const uint4*>(s_vals + off + 4 * i);
+                val[4 * i + 0] = b.x; val[4 * i + 1] = b.y; val[4 * i + 2] = b.z; val[4 * i + 3] = b.w;
+            }
+        }
+    };
+    auto none = [] {};
+    if constexpr (LOG_B > W) {
+        constexpr int W1 = LOG_B - W < W ? LOG_B - W : W;
+        reload();
+        rank_tile_pass<W, W1, NT, K, KV, FULL>(key, val, nvalid, f, s_keys, s_vals, s_cnt, s_ws, none);
+    }
+    if constexpr (LOG_B > 2 * W) {
+        constexpr int W2 = LOG_B - 2 * W;
+        static_assert(W2 <= W, "at most three passes");
+        reload();
+        rank_tile_pass<2 * W, W2, NT, K, KV, FULL>(key, val, nvalid, f, s_keys, s_vals, s_cnt, s_ws, none);
     }
 }
 

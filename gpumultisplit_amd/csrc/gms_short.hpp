@@ -24,38 +24,21 @@ struct RawF64 {
     GMS_HD uint64_t operator()(uint64_t k) const { return k; }
 };
 
-// NW consecutive words from word `off` of p, zero from word `nvalid` on.
-// `vec`: p + off may be read in 16-byte vectors.
-template <int NW>
-__device__ __forceinline__ void load_words(const uint32_t* __restrict__ p, uint32_t off,
-                                           uint32_t nvalid, bool vec, uint32_t (&x)[NW]) {
-    if (NW % 4 == 0 && vec && off + (uint32_t)NW <= nvalid) {
-#pragma unroll
-        for (int i = 0; i < NW / 4; ++i) {
-            const uint4 v = reinterpret_cast<const uint4*>(p + off)[i];
-            x[4 * i + 0] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < NW; ++i) x[i] = off + (uint32_t)i < nvalid ? p[off + i] : 0u;
-    }
-}
-
 template <int KW>
 __device__ __forceinline__ auto short_key(const uint32_t* x, int k) {
     if constexpr (KW == 2) return (uint64_t)x[2 * k] | ((uint64_t)x[2 * k + 1] << 32);
     else return x[k];
 }
 
-// Digits of the thread's elements: W bits of the id from `shift`; elements
-// past the end take the largest digit, so that they stay behind all others.
+// Digit of the thread's element k: W bits of the id from `shift`; elements past
+// the end take the largest digit, so that they stay behind all others.
 template <int W, int K, int KW, class F>
-__device__ __forceinline__ void short_digits(const uint32_t (&kx)[K * KW], uint32_t shift,
-                                             uint32_t first, uint32_t n, F f, uint32_t (&dig)[K]) {
-    constexpr uint32_t DM = (1u << W) - 1u;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-        dig[k] = first + (uint32_t)k < n ? (uint32_t)(f(short_key<KW>(kx, k)) >> shift) & DM : DM;
+__device__ __forceinline__ auto short_digit(const uint32_t (&kx)[K * KW], uint32_t shift,
+                                            uint32_t first, uint32_t n, F f) {
+    return [=, &kx](int k) {
+        constexpr uint32_t DM = (1u << W) - 1u;
+        return first + (uint32_t)k < n ? (uint32_t)(f(short_key<KW>(kx, k)) >> shift) & DM : DM;
+    };
 }
 
 // Element words in LDS: word w of element i at s[w * TILE + i].
@@ -126,9 +109,8 @@ __global__ __launch_bounds__(NT) void short_block_kernel(
     load_words<K * KW>(kin, first * KW, n * KW, vec != 0, kx);
     if constexpr (VW) load_words<K * VW>(vin, first * VW, n * VW, vec != 0, vx);
     for (uint32_t shift = 0;;) {
-        uint32_t dig[K], pos[K];
-        short_digits<4, K, KW>(kx, shift, first, n, f, dig);
-        rank_digits<4, NT, K>(dig, pos, s_cnt, s_ws, [] {});
+        uint32_t pos[K];
+        rank_digits<4, NT, K>(short_digit<4, K, KW>(kx, shift, first, n, f), pos, s_cnt, s_ws, [] {});
         short_put<K, KW, VW, TILE>(kx, vx, pos, s_item);
         __syncthreads();
         shift += 4u;
@@ -397,10 +379,9 @@ __global__ __launch_bounds__(kThreads) void short_scatter_kernel(
         }
         short_put<K, KW, VW, TILE>(kx, vx, at, s_item);
         for (uint32_t shift = 0;;) {
-            uint32_t dig[K], pos[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) dig[k] = (pk[k] >> (16u + shift)) & DM;
-            rank_digits<W, kThreads, K>(dig, pos, s_cnt, s_ws, [&] { if (shift == 0) deltas(); });
+            uint32_t pos[K];
+            rank_digits<W, kThreads, K>([&](int k) { return (pk[k] >> (16u + shift)) & DM; }, pos,
+                                        s_cnt, s_ws, [&] { if (shift == 0) deltas(); });
             short_put<K, 1, 0, TILE>(pk, none, pos, s_pk);
             __syncthreads();
             shift += (uint32_t)W;
@@ -420,9 +401,9 @@ __global__ __launch_bounds__(kThreads) void short_scatter_kernel(
         return;
     }
     for (uint32_t shift = 0;;) {
-        uint32_t dig[K], pos[K];
-        short_digits<W, K, KW>(kx, shift, first, nvalid, f, dig);
-        rank_digits<W, kThreads, K>(dig, pos, s_cnt, s_ws, [&] { if (shift == 0) deltas(); });
+        uint32_t pos[K];
+        rank_digits<W, kThreads, K>(short_digit<W, K, KW>(kx, shift, first, nvalid, f), pos, s_cnt,
+                                    s_ws, [&] { if (shift == 0) deltas(); });
         short_put<K, KW, VW, TILE>(kx, vx, pos, s_item);
         __syncthreads();
         shift += (uint32_t)W;
