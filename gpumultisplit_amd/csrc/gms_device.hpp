@@ -269,6 +269,29 @@ __device__ __forceinline__ void wait_loads() {
     __builtin_amdgcn_s_waitcnt(0);
 #endif
 }
+// 64 x 16 bytes of global memory straight into LDS: lane l's 16 bytes at g go
+// to words [4l, 4l + 4) of dst, which is the same in every lane of the wave and
+// 16-byte aligned, as g is.  No registers hold the data, and every line is read by
+// one instruction.  STREAM: not kept in the caches (ld_stream).
+// lds_loads_done() waits for them; the wave may then read what it loaded.
+template <bool STREAM>
+__device__ __forceinline__ void load_to_lds(const uint32_t* g, uint32_t* dst) {
+#ifdef GMS_HOST_EMULATION
+    __builtin_memcpy(dst + 4u * (threadIdx.x & 63u), g, 16);
+#else
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) uint32_t*)g,
+        (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, STREAM ? 2 : 0);
+#endif
+}
+__device__ __forceinline__ void lds_loads_done() {
+    wait_loads();
+#ifndef GMS_HOST_EMULATION
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#endif
+    GMS_WAVE_SYNC();
+}
+
 // Short pause in a wait loop.
 __device__ __forceinline__ void wait_pause() {
 #ifndef GMS_HOST_EMULATION

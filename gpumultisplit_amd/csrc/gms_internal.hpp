@@ -29,6 +29,10 @@ struct MsCall {
     // prescan (NULL: the scan that follows is the two-launch one).
     uint64_t* scan_status = nullptr;
     uint32_t scan_chunks = 0;
+    // The nb bucket starts, written by a postscan that writes them
+    // (reg_rank_min), or NULL.
+    uint32_t* offs = nullptr;
+    uint32_t nb = 0;
 };
 
 // Functor-family launchers (one translation unit per family).

@@ -21,6 +21,7 @@
 #pragma once
 
 #include "gms_device.hpp"
+#include "gms_rank.hpp"
 #include "gms_tune.hpp"
 
 namespace gms {
@@ -78,6 +79,9 @@ __device__ __forceinline__ void load_words(const uint32_t* __restrict__ p, uint3
             const uint4 v = reinterpret_cast<const uint4*>(p + off)[i];
             x[4 * i + 0] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
         }
+    } else if (off + (uint32_t)NW <= nvalid) {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) x[i] = p[off + i];
     } else {
 #pragma unroll
         for (int i = 0; i < NW; ++i) x[i] = off + (uint32_t)i < nvalid ? p[off + i] : 0u;
@@ -494,6 +498,15 @@ __device__ __forceinline__ uint32_t matrix_word(const uint32_t* __restrict__ m, 
     return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(m) + (off << 2));
 }
 
+// Bucket starts: the first word of each bucket's row of the scanned matrix.
+// Called last by a postscan's workgroup of tile 0.  (ms_postscan_kernel leaves them
+// to a launch of their own: the two arguments alone, a register more, cost its
+// 256-bucket form 2 %, 11 us of a sort of 2^25 pairs.)
+__device__ __forceinline__ void write_starts(const uint32_t* __restrict__ G, uint32_t num_tiles,
+                                             uint32_t* __restrict__ offs, uint32_t nb) {
+    for (uint32_t b = threadIdx.x; b < nb; b += kThreads) offs[b] = matrix_word(G, b * num_tiles);
+}
+
 // Postscan, one workgroup per tile, tiles in the XCD order (xcd_tile).  The
 // same launch shape as the prescan: on MI355X a workgroup per tile, handed
 // out by the dispatcher in tile order, measured faster than resident
@@ -578,6 +591,95 @@ __global__ __launch_bounds__(kThreads) void ms_postscan_kernel(
                                                               s_vals, s_cnt, s_delta, s_bs, s_ws);
         postscan_write<K, KV, false>(nvalid, n, kout, vout, f, s_keys, s_vals, s_delta);
     }
+}
+
+// The same with the tile loaded through LDS and ranked with register counters
+// (reg_rank_min).  The blocked loads above touch every line from K/4
+// instructions, so they need it kept in the caches between them; here a wave
+// reads its 64 * K words with 16-byte loads that each cover 1 KB of them, past
+// the caches for large inputs (STREAM), which leaves the L2 to the output lines
+// that neighbouring tiles complete.  offs: the nb bucket starts, or NULL.
+template <int LOG_B, int K, bool KV, bool VEC, bool STREAM, class F>
+__global__ __launch_bounds__(kThreads) void ms_postscan_reg_kernel(
+    const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+    uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n, uint32_t num_tiles,
+    const uint32_t* __restrict__ G, F f, uint32_t* __restrict__ offs, uint32_t nb) {
+    constexpr int B = 1 << LOG_B;
+    constexpr int W = rank_pass_bits(LOG_B);
+    constexpr uint32_t TILE = kThreads * K;
+    static_assert(B <= kThreads, "one bucket per thread");
+    __shared__ __attribute__((aligned(16))) uint32_t s_keys[TILE];
+    __shared__ __attribute__((aligned(16))) uint32_t s_vals[KV ? TILE : 4];
+    __shared__ uint32_t s_cnt[rank_cnt_words<W, kThreads>()];
+    __shared__ uint32_t s_ws[rank_ws_words<W, kThreads>()];
+    __shared__ uint32_t s_delta[B];
+    __shared__ uint32_t s_bs[kWaves];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wid = (uint32_t)GMS_READFIRSTLANE((int)(tid >> 6));
+    const uint32_t t = xcd_tile(blockIdx.x, num_tiles);
+    const uint32_t nvalid = tile_valid(n, t, TILE);
+    const size_t base = (size_t)t * TILE;
+    const bool staged = VEC && nvalid == TILE;
+    if (staged) {
+        const uint32_t w0 = wid * (64u * K);
+#pragma unroll
+        for (uint32_t j = 0; j < (uint32_t)K / 4u; ++j)
+            load_to_lds<STREAM>(kin + base + w0 + 256u * j + 4u * lane, s_keys + w0 + 256u * j);
+        if constexpr (KV) {
+#pragma unroll
+            for (uint32_t j = 0; j < (uint32_t)K / 4u; ++j)
+                load_to_lds<STREAM>(vin + base + w0 + 256u * j + 4u * lane, s_vals + w0 + 256u * j);
+        }
+    }
+    // The bucket's scanned entry and the next one in scan order (n past the
+    // end): their difference is the tile's count in the bucket.
+    const uint32_t bt = tid < (uint32_t)B ? tid : (uint32_t)B - 1u;
+    const uint32_t idx = bt * num_tiles + t;
+    const bool last = idx + 1u >= (uint32_t)B * num_tiles;
+    const uint32_t g0 = matrix_word(G, idx);
+    const uint32_t g1 = matrix_word(G, last ? idx : idx + 1u);
+    uint32_t key[K], val[K];
+    if (staged) {
+        lds_loads_done();
+        const uint4* q = reinterpret_cast<const uint4*>(s_keys + tid * (uint32_t)K);
+#pragma unroll
+        for (int i = 0; i < K / 4; ++i) {
+            const uint4 a = q[i];
+            key[4 * i + 0] = a.x; key[4 * i + 1] = a.y; key[4 * i + 2] = a.z; key[4 * i + 3] = a.w;
+        }
+        if constexpr (KV) {
+            const uint4* r = reinterpret_cast<const uint4*>(s_vals + tid * (uint32_t)K);
+#pragma unroll
+            for (int i = 0; i < K / 4; ++i) {
+                const uint4 a = r[i];
+                val[4 * i + 0] = a.x; val[4 * i + 1] = a.y; val[4 * i + 2] = a.z; val[4 * i + 3] = a.w;
+            }
+        }
+    } else {
+        load_words<K>(kin + base, tid * (uint32_t)K, nvalid, VEC, key);
+        if constexpr (KV) load_words<K>(vin + base, tid * (uint32_t)K, nvalid, VEC, val);
+    }
+    if constexpr (!KV) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) val[k] = 0;
+    }
+    const uint32_t cnt = tid < (uint32_t)B ? (last ? n : g1) - g0 : 0u;
+    const uint32_t inc = wave_incl_scan(cnt);
+    if (lane == 63u) s_bs[wid] = inc;
+    auto deltas = [&] {
+        uint32_t ls = inc - cnt;
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)kWaves; ++i) ls += i < wid ? s_bs[i] : 0u;
+        if (tid < (uint32_t)B) s_delta[tid] = g0 - ls;
+    };
+    if (nvalid == TILE) {
+        rank_tile<LOG_B, kThreads, K, KV, true>(key, val, TILE, f, s_keys, s_vals, s_cnt, s_ws, deltas);
+        postscan_write<K, KV, true>(TILE, n, kout, vout, f, s_keys, s_vals, s_delta);
+    } else {
+        rank_tile<LOG_B, kThreads, K, KV, false>(key, val, nvalid, f, s_keys, s_vals, s_cnt, s_ws, deltas);
+        postscan_write<K, KV, false>(nvalid, n, kout, vout, f, s_keys, s_vals, s_delta);
+    }
+    if (offs && t == 0) write_starts(G, num_tiles, offs, nb);
 }
 
 // ---------------------------------------------------------------------------

@@ -51,10 +51,25 @@ hipError_t launch_prescan_t(const MsCall& c, const F& f) {
 template <int LOG_B, bool KV, bool VEC, bool LARGE, class F>
 hipError_t launch_postscan_v(const MsCall& c, const F& f) {
     constexpr int K = tune_items(LOG_B, KV, LARGE);
+    const dim3 grid(c.num_tiles), block(kThreads);
+    if constexpr (reg_rank_min(LOG_B, KV) != 0) {
+        // Streamed from the size on where the prescan's loads are.
+        if (VEC && c.n >= kStreamLoadMin) {
+            hipLaunchKernelGGL((ms_postscan_reg_kernel<LOG_B, K, KV, VEC, VEC, F>), grid, block, 0,
+                               c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H, f,
+                               c.offs, c.nb);
+            return hipGetLastError();
+        }
+        if (c.n >= reg_rank_min(LOG_B, KV)) {
+            hipLaunchKernelGGL((ms_postscan_reg_kernel<LOG_B, K, KV, VEC, false, F>), grid, block,
+                               0, c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H, f,
+                               c.offs, c.nb);
+            return hipGetLastError();
+        }
+    }
     constexpr int LB = tune_level_bits(LOG_B);
-    hipLaunchKernelGGL((ms_postscan_kernel<LOG_B, K, LB, KV, VEC, F>), dim3(c.num_tiles),
-                       dim3(kThreads), 0, c.stream, c.kin, c.vin, c.kout, c.vout, c.n,
-                       c.num_tiles, c.H, f);
+    hipLaunchKernelGGL((ms_postscan_kernel<LOG_B, K, LB, KV, VEC, F>), grid, block, 0, c.stream,
+                       c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H, f);
     return hipGetLastError();
 }
 

@@ -69,6 +69,20 @@ constexpr bool tune_alias(int log_b, int items, bool kv, int level_bits) {
     return kv && cnt_row(1 << level_bits) <= items && !(log_b >= 7 && items < 28);
 }
 
+// Keys from which a class loads a postscan tile through LDS and ranks it with
+// register counters (ms_postscan_reg_kernel) instead of blocked loads and LDS
+// counters; 0: never.  On MI355X, whole call, LDS counters against registers (us):
+//   key-value  2 buckets 10M 48.7 / 47.0, 13M 60.3 / 55.9, 2^24 73.1 / 68.9, 2^25
+//              134 / 132, 2^26 240 / 238; 16 buckets 13M 66.6 / 62.0, 2^25 139 / 134,
+//              2^26 257 / 238, 90M 347 / 336; 32 buckets 20M 86.7 / 90.6, 2^26 258 / 243;
+//              64 buckets 2^26 250 / 251
+//   key-only   2 buckets 10M 29.1 / 27.5, 13M 35.7 / 32.6, 2^25 85.2 / 84.2, 2^26 143 /
+//              140; 8 buckets 13M 36.6 / 34.1, 2^26 144 / 137; 16 buckets no difference
+// At 3M to 8M keys both are the same or the LDS counters up to 5 % faster.
+constexpr uint32_t reg_rank_min(int log_b, bool kv) {
+    return log_b <= (kv ? 4 : 3) ? 9u << 20 : (kv && log_b == 5 ? kLongTileMin : 0u);
+}
+
 // Bucket counts up to this run in one prescan/scan/postscan pass (three LDS
 // ranking passes of at most 4 bits above 256); more take LSD passes over
 // 8-bit digits of the bucket id.

@@ -78,6 +78,8 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
     if (m > s.hist_cap || (!one && scan_partials_needed(m) > s.part_cap)) return GMS_ERR_CAPACITY;
     auto al16 = [](const void* p) { return p == nullptr || (((uintptr_t)p) & 15u) == 0; };
     WideCall c{kin, vin, kout, vout, n, nt, s.hist, al16(kin) && al16(vin), stream};
+    c.offs = d_offsets;
+    c.nb = B;
     if (one) {
         c.scan_status = s.status;
         c.scan_chunks = scan_chunks(m);
@@ -96,7 +98,6 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
         e = one ? launch_scan_single(s.hist, s.hist, (uint32_t)m, s.status, stream)
                 : launch_exclusive_scan(s.hist, s.hist, (uint32_t)m, s.part, stream);
     if (e == hipSuccess) e = stage(false);
-    if (e == hipSuccess && d_offsets) e = launch_gather_offsets(s.hist, nt, B, d_offsets, stream);
     return hip_status(e);
 }
 

@@ -224,7 +224,7 @@ template <int LOG_B, int K, int LEVEL_BITS, int KW, int VW, bool VEC, class F>
 __global__ __launch_bounds__(kThreads) void ms_wide_postscan_kernel(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n, uint32_t num_tiles,
-    const uint32_t* __restrict__ G, F f) {
+    const uint32_t* __restrict__ G, F f, uint32_t* __restrict__ offs, uint32_t nb) {
     constexpr int B = 1 << LOG_B;
     __shared__ __attribute__((aligned(16))) WideSmem<LOG_B, K, LEVEL_BITS, KW, VW> sm;
     const uint32_t tid = threadIdx.x;
@@ -239,6 +239,7 @@ __global__ __launch_bounds__(kThreads) void ms_wide_postscan_kernel(
     const uint32_t cntb = (idx + 1 < mtot ? g1raw : n) - g0;
     wide_postscan_item<LOG_B, K, LEVEL_BITS, KW, VW, VEC>(kin, vin, kout, vout, n, t, g0, cntb, f,
                                                           sm);
+    if (offs && t == 0) write_starts(G, num_tiles, offs, nb);
 }
 
 // ---------------------------------------------------------------- launches
@@ -256,6 +257,9 @@ struct WideCall {
     // prescan (NULL: the scan that follows is the two-launch one).
     uint64_t* scan_status = nullptr;
     uint32_t scan_chunks = 0;
+    // The nb bucket starts, written by the postscan, or NULL.
+    uint32_t* offs = nullptr;
+    uint32_t nb = 0;
 };
 
 template <int LOG_B, int KW, int VW, bool VEC, class F>
@@ -282,7 +286,7 @@ inline hipError_t wide_postscan_v(const WideCall& c, const F& f) {
     constexpr int LB = tune_level_bits(LOG_B);
     hipLaunchKernelGGL((ms_wide_postscan_kernel<LOG_B, K, LB, KW, VW, VEC, F>), dim3(c.num_tiles),
                        dim3(kThreads), 0, c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles,
-                       c.H, f);
+                       c.H, f, c.offs, c.nb);
     return hipGetLastError();
 }
 
