@@ -186,9 +186,20 @@ __global__ __launch_bounds__(kThreads) void short_count_kernel(const uint32_t* _
                 atomicAdd(&s_h[(c * B + f(short_key<KW>(y, q))) * kShortCopies + copy], 1u);
         }
     } else {
-        for (uint32_t e = tid; e < left; e += kThreads) {
-            const uint32_t c = e / TILE;
-            atomicAdd(&s_h[(c * B + f(short_key<KW>(p + (size_t)e * KW, 0))) * kShortCopies + copy], 1u);
+        // Every element on its own, all loads in flight (at the last element
+        // past the end); one ragged workgroup would otherwise set the time of all.
+        uint32_t y[C * K][KW];
+#pragma unroll
+        for (int i = 0; i < C * K; ++i) {
+            const uint32_t e = (uint32_t)i * kThreads + tid, at = e < left ? e : left - 1u;
+#pragma unroll
+            for (int w = 0; w < KW; ++w) y[i][w] = p[(size_t)at * KW + w];
+        }
+#pragma unroll
+        for (int i = 0; i < C * K; ++i) {
+            const uint32_t c = (uint32_t)i * kThreads / TILE;
+            if ((uint32_t)i * kThreads + tid < left)
+                atomicAdd(&s_h[(c * B + f(short_key<KW>(y[i], 0))) * kShortCopies + copy], 1u);
         }
     }
     __syncthreads();
@@ -234,8 +245,16 @@ __global__ __launch_bounds__(kThreads) void short_count_few_kernel(
             for (int q = 0; q < 4 / KW; ++q) c += (uint64_t)1 << (8u * f(short_key<KW>(y, q)));
         }
     } else {
-        for (uint32_t e = tid; e < nvalid; e += kThreads)
-            c += (uint64_t)1 << (8u * f(short_key<KW>(p + (size_t)e * KW, 0)));
+        uint32_t y[K][KW];
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)K; ++i) {
+            const uint32_t e = tid + i * kThreads, at = e < nvalid ? e : nvalid - 1u;
+#pragma unroll
+            for (int w = 0; w < KW; ++w) y[i][w] = p[(size_t)at * KW + w];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)K; ++i)
+            if (tid + i * kThreads < nvalid) c += (uint64_t)1 << (8u * f(short_key<KW>(y[i], 0)));
     }
     // Buckets j and j + 4 in one word.
     const uint32_t lo = (uint32_t)c, hi = (uint32_t)(c >> 32);
