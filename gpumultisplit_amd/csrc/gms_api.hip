@@ -56,11 +56,16 @@ bool ranges_overlap(const void* a, size_t an, const void* b, size_t bn) {
 // Words of the three-stage path's matrices.
 static size_t stage_matrix_elems(uint32_t n, uint32_t num_buckets) {
     if (num_buckets > 256) {
-        // 64-bit elements, and 32-bit ones above kSinglePassBuckets, take
-        // passes of at most 256 buckets; 32-bit ones up to it take one pass.
+        // 64-bit elements take passes of at most 256 buckets; 32-bit ones up to
+        // kSinglePassBuckets one pass, above it passes of at most 512.
         size_t m = stage_matrix_elems(n, 256);
-        if (num_buckets <= kSinglePassBuckets) {
-            const int lb = ceil_log2_u32(num_buckets);
+        uint32_t width[3] = {0, 0, 0};
+        int lb = ceil_log2_u32(num_buckets);
+        if (num_buckets > kSinglePassBuckets) {
+            (void)large_passes((uint32_t)lb, true, false, width);
+            lb = (int)width[0];  // the widest; key-only passes are the same or of 8 bits
+        }
+        if (lb > 8) {
             const uint32_t tko = std::min(tile_keys(lb, false, 0), tile_keys(lb, false, kLongTileMin));
             const uint32_t tkv = std::min(tile_keys(lb, true, 0), tile_keys(lb, true, kLongTileMin));
             const size_t t = std::max(((size_t)n + tko - 1) / tko, ((size_t)n + tkv - 1) / tkv);
@@ -90,6 +95,8 @@ size_t matrix_elems(uint32_t n, uint32_t num_buckets) {
                         short_matrix_words(n, std::min<uint32_t>(num_buckets, 256u)));
     if (num_buckets > 256 && num_buckets <= kSinglePassBuckets)
         m = std::max(m, short_matrix_words(n, num_buckets));
+    if (num_buckets > kSinglePassBuckets)
+        for (uint32_t w = 2; w <= 9; ++w) m = std::max(m, short_matrix_words(n, 1u << w));
     return m;
 }
 

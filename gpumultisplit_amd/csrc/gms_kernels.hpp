@@ -710,11 +710,56 @@ __global__ __launch_bounds__(kThreads) void bucket_starts_kernel(const uint32_t*
     start[b] = lo;
 }
 
+// The same with 16 lanes per bucket, which read 16 probes of the range at once:
+// log17 instead of log2 steps, each a dependent memory access.  For counts
+// that leave the chip idle (4096 buckets of 3M keys: 4.7 us, 8.4 with one lane each).
+template <int KW, class F>
+__global__ __launch_bounds__(kThreads) void bucket_starts16_kernel(const uint32_t* __restrict__ out,
+                                                                   uint32_t n, uint32_t num_buckets,
+                                                                   F f, uint32_t* __restrict__ start) {
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    const uint32_t b = i / 16u, q = i % 16u;
+    const uint32_t sub = (threadIdx.x & 48u);  // the group's first lane in the wave
+    uint32_t lo = 0, hi = b < num_buckets ? n : 0u;
+    while (GMS_BALLOT(lo < hi) != 0) {  // the same in every lane of the wave
+        const uint32_t len = hi - lo;
+        // up to 16 elements: all of them; else 16 that cut the range in 17
+        const uint32_t at = len <= 16u ? lo + q : lo + (uint32_t)((uint64_t)(q + 1u) * len / 17u);
+        bool below = false;
+        if (at < hi) {
+            uint32_t id;
+            if constexpr (KW == 2)
+                id = f((uint64_t)out[2 * (size_t)at] | ((uint64_t)out[2 * (size_t)at + 1] << 32));
+            else
+                id = f(out[at]);
+            below = id < b;
+        }
+        const uint32_t c = (uint32_t)__builtin_popcountll((GMS_BALLOT(below) >> sub) & 0xFFFFull);
+        // c probes lie below bucket b: its start is behind the last of them and
+        // not behind the next one.
+        const uint32_t l = lo;
+        if (len <= 16u) {
+            lo = l + c;
+            hi = lo;
+        } else {
+            if (c) lo = l + (uint32_t)((uint64_t)c * len / 17u) + 1u;
+            if (c < 16u) hi = l + (uint32_t)((uint64_t)(c + 1u) * len / 17u);
+        }
+    }
+    if (q == 0 && b < num_buckets) start[b] = lo;
+}
+
 template <int KW, class F>
 hipError_t launch_bucket_starts(const uint32_t* out, uint32_t n, uint32_t num_buckets, const F& f,
                                 uint32_t* start, hipStream_t stream) {
-    hipLaunchKernelGGL((bucket_starts_kernel<KW, F>), dim3((num_buckets + kThreads - 1) / kThreads),
-                       dim3(kThreads), 0, stream, out, n, num_buckets, f, start);
+    const uint32_t per = num_buckets <= 16384u ? 16u : 1u;  // lanes per bucket
+    const dim3 grid((num_buckets * per + kThreads - 1) / kThreads);
+    if (per == 16u)
+        hipLaunchKernelGGL((bucket_starts16_kernel<KW, F>), grid, dim3(kThreads), 0, stream, out, n,
+                           num_buckets, f, start);
+    else
+        hipLaunchKernelGGL((bucket_starts_kernel<KW, F>), grid, dim3(kThreads), 0, stream, out, n,
+                           num_buckets, f, start);
     return hipGetLastError();
 }
 

@@ -133,12 +133,12 @@ gms_status run_wide_large(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint
         if (e != hipSuccess || !d_offsets || offs) return hip_status(e);
         return wide_starts(kout, n, kw, B, d, d_offsets, stream);
     }
-    const int passes = (bits + 7) / 8;
+    uint32_t width[3], shift = 0;
+    const int passes = large_passes((uint32_t)bits, vw != 0, true, width);
     const uint32_t* sk = kin;
     const uint32_t* sv = vin;
-    for (int p = 0; p < passes; ++p) {
-        const uint32_t shift = 8u * (uint32_t)p;
-        const uint32_t w = (uint32_t)(bits - (int)shift < 8 ? bits - (int)shift : 8);
+    for (int p = 0; p < passes; shift += width[p++]) {
+        const uint32_t w = width[p];
         const bool to_out = ((passes - 1 - p) % 2) == 0;  // the last pass writes the output
         uint32_t* dk = to_out ? kout : ktmp;
         uint32_t* dv = vw ? (to_out ? vout : vtmp) : nullptr;

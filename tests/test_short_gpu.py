@@ -141,3 +141,28 @@ def test_host_results_of_many_contexts(dev, B):
         np.testing.assert_array_equal(from_dev(kout)[:n], wk)
         for c in ctxs:
             gms.multisplit_release_memory(c)
+
+
+@pytest.mark.parametrize("kv", [False, True])
+@pytest.mark.parametrize("B", [2048, 4096, 5000, 100_000, 200_000, 500_000, 1 << 20])
+def test_many_buckets_pass_widths(dev, B, kv):
+    """Bucket counts of 11, 12, 13, 17, 18, 19 and 20 bits, whose LSD passes have
+    different widths, below and above the two-launch sizes, with the starts of
+    both search kernels."""
+    ctx = gms.multisplit_context(B)
+    gms.multisplit_allocate_key_value(2_200_001, ctx)
+    for n in (8193, 300_007, 2_200_001):
+        banner(f"many buckets B={B} kv={kv} n={n}")
+        keys = W.uniform_keys(n, seed=B + n)
+        keys[:n // 7] = keys[0]
+        vals = np.arange(n, dtype=np.uint32)
+        kout, vout = filled_u32(n, dev), filled_u32(n, dev) if kv else None
+        offs = filled_u32(B, dev, 0xFFFFFFFF)
+        gms.multisplit(to_dev(keys, dev), kout, n, ctx, gms.range_bucket(B),
+                       d_value_in=to_dev(vals, dev) if kv else None, d_value_out=vout,
+                       d_offsets=offs)
+        wk, wv, wo = oracle.multisplit(keys, B, oracle.RANGE, 0, vals if kv else None)
+        np.testing.assert_array_equal(from_dev(kout)[:n], wk)
+        np.testing.assert_array_equal(from_dev(offs), wo)
+        if kv:
+            np.testing.assert_array_equal(from_dev(vout)[:n], wv)
