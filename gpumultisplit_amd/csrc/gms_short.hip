@@ -34,8 +34,14 @@ hipError_t block_shape(const ShortCall& c, uint32_t bits, const F& f) {
             if (e != hipSuccess) return e;
         }
     }
+    // Sorts of 32-bit keys, us: 2000 keys 512 x 4 9.5, 1024 x 4 15.0; 4000 keys 512 x
+    // 8 13.0, 1024 x 4 16.4; 5003 keys 512 x 12 16.8, 1024 x 8 20.9; 8000 keys 512 x
+    // 16 22.5, 1024 x 8 21.4 (a pass's wave scans cost every wave the same, however
+    // few its keys).
     if (c.n <= 1024u) return block_t<256, 4, KW, VW>(c, bits, f);
-    if (c.n <= 4096u) return block_t<1024, 4, KW, VW>(c, bits, f);
+    if (c.n <= 2048u) return block_t<512, 4, KW, VW>(c, bits, f);
+    if (c.n <= 4096u) return block_t<512, 8, KW, VW>(c, bits, f);
+    if (c.n <= 6144u) return block_t<512, 12, KW, VW>(c, bits, f);
     return block_t<1024, 8, KW, VW>(c, bits, f);
 }
 
@@ -115,10 +121,10 @@ hipError_t two_shape(const ShortCall& c, const ShortPlan& p, uint32_t* H, const 
 //   256 buckets  1k 4.6 / 6.7 us, 4k 6.6 / 7.4, 8k 9.0 / 7.6
 //   1024 buckets 1k 7.8 / 8.1 us, 4k 9.1 / 8.8, 8k 12.4 / 9.2
 // so up to 8192 elements, but 4096 where the ids have 9 to 12 bits (a sort's
-// 32-bit ids would take four times two launches instead) and where four words
-// per element leave no LDS for more.
+// 32-bit ids would take four times two launches instead), and 6144 where four
+// words per element leave no LDS for more.
 bool short_one_block(uint32_t n, uint32_t bits, uint32_t kw, uint32_t vw) {
-    return n <= (kw + vw > 3u || (bits > 8u && bits <= 12u) ? 4096u : 8192u);
+    return n <= (bits > 8u && bits <= 12u ? 4096u : kw + vw > 3u ? 6144u : 8192u);
 }
 
 // Tiles of 4 elements per thread while that gives at most one tile per CU,

@@ -14,7 +14,7 @@ from gpu_util import banner, filled_u32, from_dev, to_dev
 
 pytestmark = pytest.mark.gpu
 
-EDGES = (1, 1023, 1024, 1025, 4095, 4096, 4097, 8192, 8193)
+EDGES = (1, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097, 6144, 6145, 8192, 8193)
 
 
 def _around(*sizes):
