@@ -166,3 +166,22 @@ def test_many_buckets_pass_widths(dev, B, kv):
         np.testing.assert_array_equal(from_dev(offs), wo)
         if kv:
             np.testing.assert_array_equal(from_dev(vout)[:n], wv)
+
+
+@pytest.mark.gpu
+def test_stream_and_pointer_of_tensors(dev):
+    """The stream a call goes to is the current one of the tensor's device, for
+    plain tensors and subclasses alike; what was refused stays refused."""
+    import torch
+    t = torch.zeros(8, dtype=torch.int32, device=dev)
+    sub = torch.nn.Parameter(t, requires_grad=False)
+    side = torch.cuda.Stream()
+    for _ in range(2):
+        for stream in (torch.cuda.default_stream(), side):
+            with torch.cuda.stream(stream):
+                assert gms._stream(None, t) == stream.cuda_stream
+                assert gms._stream(sub) == stream.cuda_stream
+    assert gms._ptr(t) == gms._ptr(sub) == t.data_ptr()
+    for bad in (t[::2], t.cpu(), t.to(torch.int64), t.to(torch.int16)):
+        with pytest.raises(ValueError):
+            gms._ptr(bad)
