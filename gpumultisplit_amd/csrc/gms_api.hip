@@ -355,9 +355,8 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
     MsCall c;
     gms_status st = plan_call(s, kin, vin, kout, vout, n, B, kv, stream, c);
     if (st != GMS_SUCCESS) return st;
-    const uint32_t reg_min = reg_rank_min(c.log_b, kv);
-    const bool postscan_starts = reg_min != 0 && n >= reg_min;
-    if (postscan_starts) {
+    c.reg_rank = reg_rank(c.log_b, kv, n, d_offsets != nullptr);
+    if (c.reg_rank) {
         c.offs = d_offsets;
         c.nb = B;
     }
@@ -371,7 +370,7 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
     if (e == hipSuccess && ev) e = hipEventRecord(ev[2], stream);
     if (e == hipSuccess) e = with_f([&](auto f) { return launch_postscan(c, f); });
     if (e == hipSuccess && ev) e = hipEventRecord(ev[3], stream);
-    if (e == hipSuccess && d_offsets && !postscan_starts)
+    if (e == hipSuccess && d_offsets && !c.reg_rank)
         e = launch_gather_offsets(s.hist, c.num_tiles, B, d_offsets, stream);
     return hip_status(e);
 }

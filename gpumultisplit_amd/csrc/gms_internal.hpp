@@ -29,8 +29,9 @@ struct MsCall {
     // prescan (NULL: the scan that follows is the two-launch one).
     uint64_t* scan_status = nullptr;
     uint32_t scan_chunks = 0;
-    // The nb bucket starts, written by a postscan that writes them
-    // (reg_rank_min), or NULL.
+    // Whether the postscan is the register-counter one (reg_rank), and the nb
+    // bucket starts that it then writes, or NULL.
+    bool reg_rank = false;
     uint32_t* offs = nullptr;
     uint32_t nb = 0;
 };

@@ -594,7 +594,7 @@ __global__ __launch_bounds__(kThreads) void ms_postscan_kernel(
 }
 
 // The same with the tile loaded through LDS and ranked with register counters
-// (reg_rank_min).  The blocked loads above touch every line from K/4
+// (reg_rank).  The blocked loads above touch every line from K/4
 // instructions, so they need it kept in the caches between them; here a wave
 // reads its 64 * K words with 16-byte loads that each cover 1 KB of them, past
 // the caches for large inputs (STREAM), which leaves the L2 to the output lines

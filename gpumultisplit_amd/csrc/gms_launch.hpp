@@ -52,17 +52,20 @@ template <int LOG_B, bool KV, bool VEC, bool LARGE, class F>
 hipError_t launch_postscan_v(const MsCall& c, const F& f) {
     constexpr int K = tune_items(LOG_B, KV, LARGE);
     const dim3 grid(c.num_tiles), block(kThreads);
-    if constexpr (reg_rank_min(LOG_B, KV) != 0) {
-        // Streamed from the size on where the prescan's loads are.
-        if (VEC && c.n >= kStreamLoadMin) {
-            hipLaunchKernelGGL((ms_postscan_reg_kernel<LOG_B, K, KV, VEC, VEC, F>), grid, block, 0,
-                               c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H, f,
-                               c.offs, c.nb);
-            return hipGetLastError();
+    // A shape of its own for large inputs (LARGE) has no register form.
+    if constexpr (!LARGE && reg_rank_starts_below(LOG_B, KV) != 0) {
+        if constexpr (VEC && reg_rank_from(LOG_B, KV) != 0) {
+            // Streamed from the size on where the prescan's loads are.
+            if (c.reg_rank && c.n >= kStreamLoadMin) {
+                hipLaunchKernelGGL((ms_postscan_reg_kernel<LOG_B, K, KV, true, true, F>), grid, block,
+                                   0, c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H,
+                                   f, c.offs, c.nb);
+                return hipGetLastError();
+            }
         }
-        if (c.n >= reg_rank_min(LOG_B, KV)) {
-            hipLaunchKernelGGL((ms_postscan_reg_kernel<LOG_B, K, KV, VEC, false, F>), grid, block,
-                               0, c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H, f,
+        if (c.reg_rank) {
+            hipLaunchKernelGGL((ms_postscan_reg_kernel<LOG_B, K, KV, VEC, false, F>), grid, block, 0,
+                               c.stream, c.kin, c.vin, c.kout, c.vout, c.n, c.num_tiles, c.H, f,
                                c.offs, c.nb);
             return hipGetLastError();
         }

@@ -69,18 +69,41 @@ constexpr bool tune_alias(int log_b, int items, bool kv, int level_bits) {
     return kv && cnt_row(1 << level_bits) <= items && !(log_b >= 7 && items < 28);
 }
 
-// Keys from which a class loads a postscan tile through LDS and ranks it with
-// register counters (ms_postscan_reg_kernel) instead of blocked loads and LDS
-// counters; 0: never.  On MI355X, whole call, LDS counters against registers (us):
+// Keys from which a class always loads a postscan tile through LDS and ranks it
+// with register counters (ms_postscan_reg_kernel) instead of blocked loads and
+// LDS counters; 0: no such size.  On MI355X, whole call, LDS counters against
+// registers (us):
 //   key-value  2 buckets 10M 48.7 / 47.0, 13M 60.3 / 55.9, 2^24 73.1 / 68.9, 2^25
 //              134 / 132, 2^26 240 / 238; 16 buckets 13M 66.6 / 62.0, 2^25 139 / 134,
-//              2^26 257 / 238, 90M 347 / 336; 32 buckets 20M 86.7 / 90.6, 2^26 258 / 243;
-//              64 buckets 2^26 250 / 251
+//              2^26 257 / 238, 90M 347 / 336; 32 buckets 20M 86.7 / 90.6, 2^26 258 / 243
 //   key-only   2 buckets 10M 29.1 / 27.5, 13M 35.7 / 32.6, 2^25 85.2 / 84.2, 2^26 143 /
-//              140; 8 buckets 13M 36.6 / 34.1, 2^26 144 / 137; 16 buckets no difference
-// At 3M to 8M keys both are the same or the LDS counters up to 5 % faster.
-constexpr uint32_t reg_rank_min(int log_b, bool kv) {
+//              140; 8 buckets 13M 36.6 / 34.1, 2^26 144 / 137
+// At 3M to 8M keys both are the same or the LDS counters up to 5 % faster.  With
+// more buckets it depends on the identifier and on what wrote the input: 2^25 pairs
+// in 256 buckets 157 / 149 by range but 153 / 154 by division, passes of an 8-bit
+// sort of 2^25 keys 98 / 107, of 2^26 pairs 277 / 413.
+constexpr uint32_t reg_rank_from(int log_b, bool kv) {
     return log_b <= (kv ? 4 : 3) ? 9u << 20 : (kv && log_b == 5 ? kLongTileMin : 0u);
+}
+
+// Keys below which it does so in a call that wants the bucket starts: this form
+// writes them, the other leaves them to a launch of about 4 us and the gap before
+// it.  Range / division / digit identifier, as above:
+//   key-only   16 buckets 2.2M 19.9 / 18.2, 21.8 / 20.1, 20.8 / 18.7; 64 buckets 6M
+//              27.2 / 23.5, 29.5 / 26.1, 27.4 / 24.9, at 9.5M 35.9 / 32.6, 39.2 / 37.5,
+//              36.5 / 35.8, at 24M by digit 63 / 68; 256 buckets 4M 27.8 / 23.3, 29.6 /
+//              25.9, 28.4 / 25.0
+//   key-value  2 buckets 4M 24.9 / 18.9 by range, 8M 32.8 / 31.2; 16 buckets 6M 35.6 /
+//              34.2, 36.0 / 35.1, 35.5 / 34.0; 64 buckets 6M 34.5 / 32.7, 36.0 / 34.9,
+//              34.7 / 33.0, at 9.5M 44.1 / 45.3, 46.8 / 48.8, 45.1 / 45.4; 256 buckets 6M
+//              42.4 / 37.0, 43.9 / 38.9, 42.9 / 36.6
+constexpr uint32_t reg_rank_starts_below(int log_b, bool kv) {
+    return log_b > 8 ? 0u : (kv && log_b > 3 ? 7u << 20 : 9u << 20);
+}
+
+constexpr bool reg_rank(int log_b, bool kv, uint32_t n, bool starts) {
+    const uint32_t from = reg_rank_from(log_b, kv);
+    return (from && n >= from) || (starts && n < reg_rank_starts_below(log_b, kv));
 }
 
 // Bucket counts up to this run in one prescan/scan/postscan pass (three LDS
