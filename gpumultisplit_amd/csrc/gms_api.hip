@@ -53,6 +53,13 @@ bool ranges_overlap(const void* a, size_t an, const void* b, size_t bn) {
     return a0 < b1 && b0 < a1;
 }
 
+bool starts_apart(const uint32_t* offs, uint32_t nb, const uint32_t* kin, const uint32_t* vin,
+                  const uint32_t* kout, const uint32_t* vout, uint32_t n, uint32_t kw, uint32_t vw) {
+    const size_t ob = (size_t)nb * 4, kb = (size_t)n * kw * 4, vb = (size_t)n * vw * 4;
+    return !ranges_overlap(offs, ob, kin, kb) && !ranges_overlap(offs, ob, kout, kb) &&
+           !ranges_overlap(offs, ob, vin, vb) && !ranges_overlap(offs, ob, vout, vb);
+}
+
 // Words of the three-stage path's matrices.
 static size_t stage_matrix_elems(uint32_t n, uint32_t num_buckets) {
     if (num_buckets > 256) {
@@ -343,9 +350,10 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
         return hip_status(e);
     }
     const uint32_t bits = (uint32_t)ceil_log2_u32(B);
+    const bool apart = starts_apart(d_offsets, B, kin, vin, kout, vout, n, 1, kv);
     const bool block = short_one_block(n, bits, 1, kv);
     const ShortPlan sp = short_plan(n, B, 1, kv);
-    if (block || (sp.items && sp.matrix_words <= s.hist_cap)) {
+    if (apart && (block || (sp.items && sp.matrix_words <= s.hist_cap))) {
         hipEvent_t* ev = (prof && prof->on) ? prof->next(stream) : nullptr;
         const ShortCall c{kin, vin, kout, vout, n, 1u, kv ? 1u : 0u, d_offsets, B, stream, ev};
         hipError_t e = block ? launch_short_block(c, bits, any) : launch_short_two(c, sp, s.hist, any);
@@ -355,8 +363,8 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
     MsCall c;
     gms_status st = plan_call(s, kin, vin, kout, vout, n, B, kv, stream, c);
     if (st != GMS_SUCCESS) return st;
-    c.reg_rank = reg_rank(c.log_b, kv, n, d_offsets != nullptr);
-    if (c.reg_rank) {
+    c.reg_rank = reg_rank(c.log_b, kv, n, d_offsets && apart);
+    if (c.reg_rank && apart) {
         c.offs = d_offsets;
         c.nb = B;
     }
@@ -370,7 +378,7 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
     if (e == hipSuccess && ev) e = hipEventRecord(ev[2], stream);
     if (e == hipSuccess) e = with_f([&](auto f) { return launch_postscan(c, f); });
     if (e == hipSuccess && ev) e = hipEventRecord(ev[3], stream);
-    if (e == hipSuccess && d_offsets && !c.reg_rank)
+    if (e == hipSuccess && d_offsets && !c.offs)
         e = launch_gather_offsets(s.hist, c.num_tiles, B, d_offsets, stream);
     return hip_status(e);
 }

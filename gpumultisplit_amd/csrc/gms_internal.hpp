@@ -237,5 +237,12 @@ hipError_t launch_short_two(const ShortCall& c, const ShortPlan& p, uint32_t* H,
 
 gms_status hip_status(hipError_t e);
 bool ranges_overlap(const void* a, size_t an, const void* b, size_t bn);
+// Whether the nb bucket starts (NULL: none) share no word with the n elements of kw key and vw
+// value words that a call reads and writes.  Starts written by the kernel that also scatters
+// the elements need that: others of its workgroups may still read the input, or write the
+// output, when one hands out the starts.  Where they do share words, the starts come from a
+// launch of their own, behind the last read of the input.
+bool starts_apart(const uint32_t* offs, uint32_t nb, const uint32_t* kin, const uint32_t* vin,
+                  const uint32_t* kout, const uint32_t* vout, uint32_t n, uint32_t kw, uint32_t vw);
 
 }  // namespace gms

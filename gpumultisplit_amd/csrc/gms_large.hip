@@ -71,7 +71,9 @@ gms_status run_large_multisplit(LargeScratch& L, Scratch& s, const uint32_t* kin
     const bool kv = vin != nullptr;
     const int bits = ceil_log2_u32(B);
     if (short_one_block(n, (uint32_t)bits, 1, kv)) {
-        uint32_t* offs = B <= kShortBlockOffsets ? d_offsets : nullptr;
+        uint32_t* offs = B <= kShortBlockOffsets &&
+                                 starts_apart(d_offsets, B, kin, vin, kout, vout, n, 1, kv)
+                             ? d_offsets : nullptr;
         const ShortCall c{kin, vin, kout, vout, n, 1u, kv ? 1u : 0u, offs, B, stream};
         const hipError_t e = launch_short_block(c, (uint32_t)bits, DigitOfF{base, 0u, ~0u});
         if (e != hipSuccess || !d_offsets || offs) return hip_status(e);

@@ -60,9 +60,10 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
     }
     const int lb = ceil_log2_u32(B);
     // Short inputs: one or two launches.
+    const bool apart = starts_apart(d_offsets, B, kin, vin, kout, vout, n, kw, vw);
     const bool block = short_one_block(n, (uint32_t)lb, kw, vw);
     const ShortPlan sp = short_plan(n, B, kw, vw);
-    if (block || (sp.items && sp.matrix_words <= s.hist_cap)) {
+    if (apart && (block || (sp.items && sp.matrix_words <= s.hist_cap))) {
         const ShortCall c{kin, vin, kout, vout, n, kw, vw, d_offsets, B, stream};
         auto go = [&](const auto& f) {
             return block ? launch_short_block(c, (uint32_t)lb, f) : launch_short_two(c, sp, s.hist, f);
@@ -78,7 +79,7 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
     if (m > s.hist_cap || (!one && scan_partials_needed(m) > s.part_cap)) return GMS_ERR_CAPACITY;
     auto al16 = [](const void* p) { return p == nullptr || (((uintptr_t)p) & 15u) == 0; };
     WideCall c{kin, vin, kout, vout, n, nt, s.hist, al16(kin) && al16(vin), stream};
-    c.offs = d_offsets;
+    c.offs = apart ? d_offsets : nullptr;
     c.nb = B;
     if (one) {
         c.scan_status = s.status;
@@ -98,6 +99,8 @@ static gms_status wide_stages(Scratch& s, const uint32_t* kin, const uint32_t* v
         e = one ? launch_scan_single(s.hist, s.hist, (uint32_t)m, s.status, stream)
                 : launch_exclusive_scan(s.hist, s.hist, (uint32_t)m, s.part, stream);
     if (e == hipSuccess) e = stage(false);
+    if (e == hipSuccess && d_offsets && !c.offs)
+        e = launch_gather_offsets(s.hist, nt, B, d_offsets, stream);
     return hip_status(e);
 }
 
@@ -126,7 +129,9 @@ gms_status run_wide_large(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint
     if (n == 0) return d_offsets ? hip_status(launch_fill(d_offsets, 0u, B, stream)) : GMS_SUCCESS;
     const int bits = ceil_log2_u32(B);
     if (short_one_block(n, (uint32_t)bits, kw, vw)) {
-        uint32_t* offs = B <= kShortBlockOffsets ? d_offsets : nullptr;
+        uint32_t* offs = B <= kShortBlockOffsets &&
+                                 starts_apart(d_offsets, B, kin, vin, kout, vout, n, kw, vw)
+                             ? d_offsets : nullptr;
         const ShortCall c{kin, vin, kout, vout, n, kw, vw, offs, B, stream};
         auto go = [&](const auto& f) { return launch_short_block(c, (uint32_t)bits, f); };
         const hipError_t e = kw == 2 ? with_id64(d, B, 0u, ~0u, go) : go(id32(d, B, 0u, ~0u));
