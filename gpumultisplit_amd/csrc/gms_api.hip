@@ -175,8 +175,10 @@ uint32_t* pinned_results(Scratch& s) {
     std::lock_guard<std::mutex> lk(g_pinned_mu);
     PinnedBlock& b = g_pinned[s.device];
     if (!b.base && hipHostMalloc((void**)&b.base, 64u * kPinnedResults * sizeof(uint32_t),
-                                 hipHostMallocDefault) != hipSuccess)
+                                 hipHostMallocDefault) != hipSuccess) {
         b.base = nullptr;
+        (void)hipGetLastError();  // else the call's launches would report it as theirs
+    }
     if (!b.base || b.used == ~0ull) return nullptr;
     const int slot = __builtin_ctzll(~b.used);
     b.used |= 1ull << slot;

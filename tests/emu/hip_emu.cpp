@@ -193,7 +193,12 @@ void launch(dim3 grid, dim3 block, std::function<void()> body) {
 }
 
 std::atomic<uint64_t> alloc_calls{0};
+std::atomic<uint32_t> refuse_pinned{0};
+thread_local int last_error = 0;
 }  // namespace gms_emu
 
 // Allocation calls (hipMalloc, hipFree, hipHostMalloc, hipHostFree) so far.
 extern "C" uint64_t gms_emu_alloc_calls() { return gms_emu::alloc_calls.load(); }
+
+// The next `count` pinned allocations fail.
+extern "C" void gms_emu_refuse_pinned(uint32_t count) { gms_emu::refuse_pinned = count; }

@@ -121,6 +121,11 @@ inline hipError_t hipGetDevice(int* d) {
 namespace gms_emu {
 // Device and pinned allocations and frees made so far (gms_emu_alloc_calls).
 extern std::atomic<uint64_t> alloc_calls;
+// Pinned allocations still to be refused (gms_emu_refuse_pinned).
+extern std::atomic<uint32_t> refuse_pinned;
+// The last error of a runtime call of this thread, handed out and cleared by
+// hipGetLastError; a later call that succeeds leaves it, as in the HIP runtime.
+extern thread_local int last_error;
 }
 // A __device__ variable is a host global here: its address is the device one.
 #define HIP_SYMBOL(x) reinterpret_cast<const void*>(&(x))
@@ -156,7 +161,11 @@ inline hipError_t hipMemcpy(void* d, const void* s, size_t b, hipMemcpyKind) {
 }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
-inline hipError_t hipGetLastError() { return hipSuccess; }
+inline hipError_t hipGetLastError() {
+    const hipError_t e = (hipError_t)gms_emu::last_error;
+    gms_emu::last_error = hipSuccess;
+    return e;
+}
 inline hipError_t hipEventCreate(hipEvent_t* e) {
     *e = new gms_emu_event();
     return hipSuccess;
@@ -184,6 +193,12 @@ inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
 #define hipHostMallocDefault 0u
 inline hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
     ++gms_emu::alloc_calls;
+    if (gms_emu::refuse_pinned != 0) {
+        --gms_emu::refuse_pinned;
+        gms_emu::last_error = hipErrorOutOfMemory;
+        *p = nullptr;
+        return hipErrorOutOfMemory;
+    }
     *p = aligned_alloc(256, ((bytes + 255) / 256) * 256);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
