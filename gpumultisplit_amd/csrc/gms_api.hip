@@ -107,13 +107,68 @@ size_t matrix_elems(uint32_t n, uint32_t num_buckets) {
     return m;
 }
 
-static void give_back_pinned(Scratch& s);
+// Host results are written by the kernels into pinned memory and read there
+// after the stream is synchronised: a copy to the caller's pageable array,
+// staged by the runtime, costs 11 us more (launch, copy and synchronisation
+// 22.6 us on MI355X against 11.5 us).  Pinning a page takes 10 to 30 us, so the
+// contexts of a device share one block of slots, allocated with the first of
+// them and freed with the last: a call itself allocates nothing, as another
+// thread may be capturing a graph.  A context takes a slot with its first call
+// that wants host results; with every slot taken (64 contexts), or where the
+// block could not be had, the call falls back to the copy.
+namespace {
+constexpr int kPinnedDevices = 64;
+struct PinnedBlock {
+    uint32_t* base = nullptr;
+    uint64_t used = 0;      // one bit per slot
+    uint32_t contexts = 0;  // that may take one
+};
+std::mutex g_pinned_mu;
+PinnedBlock g_pinned[kPinnedDevices];
+}  // namespace
 
-gms_status scratch_alloc(Scratch& s, size_t hist_elems) {
-    scratch_free(s);
+static void join_pinned(int device) {
+    if (device < 0 || device >= kPinnedDevices) return;
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    PinnedBlock& b = g_pinned[device];
+    if (b.contexts++ == 0 && hipHostMalloc((void**)&b.base, 64u * kPinnedResults * sizeof(uint32_t),
+                                           hipHostMallocDefault) != hipSuccess) {
+        b.base = nullptr;
+        (void)hipGetLastError();  // else the next launch would report it as its own
+    }
+}
+
+static void leave_pinned(int device, uint32_t* slot) {
+    if (device < 0 || device >= kPinnedDevices) return;
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    PinnedBlock& b = g_pinned[device];
+    if (slot) b.used &= ~(1ull << ((size_t)(slot - b.base) / kPinnedResults));
+    if (--b.contexts == 0 && b.base) {
+        (void)hipHostFree(b.base);
+        b.base = nullptr;
+    }
+}
+
+uint32_t* pinned_results(Scratch& s) {
+    if (s.pin || !s.host_results || s.device < 0 || s.device >= kPinnedDevices) return s.pin;
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    PinnedBlock& b = g_pinned[s.device];
+    if (!b.base || b.used == ~0ull) return nullptr;
+    const int slot = __builtin_ctzll(~b.used);
+    b.used |= 1ull << slot;
+    s.pin = b.base + (size_t)slot * kPinnedResults;
+    return s.pin;
+}
+
+gms_status scratch_alloc(Scratch& s, size_t hist_elems, bool host_results) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return GMS_ERR_NO_DEVICE;
+    const hipError_t have = hipGetDevice(&dev);
+    // joined before the former scratch leaves, so that its last context keeps the block
+    if (have == hipSuccess && host_results) join_pinned(dev);
+    scratch_free(s);
+    if (have != hipSuccess) return GMS_ERR_NO_DEVICE;
     s.device = dev;
+    s.host_results = host_results;
     const size_t he = std::max<size_t>(hist_elems, 4);
     const size_t pe = scan_partials_needed(he);
     if (hipMalloc((void**)&s.hist, he * sizeof(uint32_t)) != hipSuccess) {
@@ -147,55 +202,12 @@ void scratch_free(Scratch& s) {
     if (s.part) (void)hipFree(s.part);
     if (s.offs) (void)hipFree(s.offs);
     if (s.status) (void)hipFree(s.status);
-    give_back_pinned(s);
+    if (s.host_results) leave_pinned(s.device, s.pin);
+    s.host_results = false;
+    s.pin = nullptr;
     s.hist = s.part = s.offs = nullptr;
     s.status = nullptr;
     s.hist_cap = s.part_cap = s.status_cap = 0;
-}
-
-// Host results are written by the kernels into pinned memory and read there
-// after the stream is synchronised: a copy to the caller's pageable array,
-// staged by the runtime, costs 11 us more (launch, copy and synchronisation
-// 22.6 us on MI355X against 11.5 us).  Pinning a page takes 10 to 30 us, so the
-// contexts of a device share one block of slots: it is allocated when the first
-// of them needs a slot and freed when the last one gives its slot back.  With
-// every slot taken (64 contexts), a call falls back to the copy.
-namespace {
-constexpr int kPinnedDevices = 64;
-struct PinnedBlock {
-    uint32_t* base = nullptr;
-    uint64_t used = 0;  // one bit per slot
-};
-std::mutex g_pinned_mu;
-PinnedBlock g_pinned[kPinnedDevices];
-}  // namespace
-
-uint32_t* pinned_results(Scratch& s) {
-    if (s.pin || s.device < 0 || s.device >= kPinnedDevices) return s.pin;
-    std::lock_guard<std::mutex> lk(g_pinned_mu);
-    PinnedBlock& b = g_pinned[s.device];
-    if (!b.base && hipHostMalloc((void**)&b.base, 64u * kPinnedResults * sizeof(uint32_t),
-                                 hipHostMallocDefault) != hipSuccess) {
-        b.base = nullptr;
-        (void)hipGetLastError();  // else the call's launches would report it as theirs
-    }
-    if (!b.base || b.used == ~0ull) return nullptr;
-    const int slot = __builtin_ctzll(~b.used);
-    b.used |= 1ull << slot;
-    s.pin = b.base + (size_t)slot * kPinnedResults;
-    return s.pin;
-}
-
-static void give_back_pinned(Scratch& s) {
-    if (!s.pin) return;
-    std::lock_guard<std::mutex> lk(g_pinned_mu);
-    PinnedBlock& b = g_pinned[s.device];
-    b.used &= ~(1ull << ((size_t)(s.pin - b.base) / kPinnedResults));
-    s.pin = nullptr;
-    if (b.used == 0) {
-        (void)hipHostFree(b.base);
-        b.base = nullptr;
-    }
 }
 
 hipEvent_t* Profiler::next(hipStream_t) {
@@ -614,7 +626,7 @@ gms_status gms_multisplit_allocate(gms_multisplit_ctx* ctx, uint32_t n_capacity,
     // drops them, and the next call that needs them allocates them anew.
     free_wide_temporaries(ctx);
     const bool large = ctx->num_buckets > 256;
-    gms_status st = scratch_alloc(ctx->s, matrix_elems(n_capacity, ctx->num_buckets));
+    gms_status st = scratch_alloc(ctx->s, matrix_elems(n_capacity, ctx->num_buckets), true);
     if (st == GMS_SUCCESS && large)
         st = large_scratch_alloc(ctx->large, n_capacity, ctx->num_buckets,
                                  ctx->num_buckets > kSinglePassBuckets);
@@ -976,7 +988,7 @@ gms_status gms_sort_allocate(gms_sort_ctx* ctx, uint32_t n_capacity, uint32_t di
     gms_sort_release(ctx);
     size_t me = 0;
     for (int i = 0; i < np; ++i) me = std::max(me, matrix_elems(n_capacity, 1u << p[i].bits));
-    gms_status st = scratch_alloc(ctx->s, me);
+    gms_status st = scratch_alloc(ctx->s, me, false);
     if (st != GMS_SUCCESS) return st;
     const size_t bytes = std::max<size_t>((size_t)n_capacity, 1) * sizeof(uint32_t);
     if (hipMalloc((void**)&ctx->ktmp, bytes) != hipSuccess) {
@@ -1010,7 +1022,7 @@ gms_status gms_sort_allocate_wide(gms_sort_ctx* ctx, uint32_t n_capacity, uint32
     gms_sort_release(ctx);
     size_t me = 0;
     for (int i = 0; i < np; ++i) me = std::max(me, matrix_elems(n_capacity, 1u << p[i].bits));
-    gms_status st = scratch_alloc(ctx->s, me);
+    gms_status st = scratch_alloc(ctx->s, me, false);
     if (st != GMS_SUCCESS) return st;
     const size_t words = std::max<size_t>((size_t)n_capacity, 1);
     if (hipMalloc((void**)&ctx->ktmp, words * kw * sizeof(uint32_t)) != hipSuccess) {
@@ -1123,7 +1135,7 @@ gms_status gms_compaction_create(gms_compaction_ctx** out) {
 gms_status gms_compaction_allocate(gms_compaction_ctx* ctx, uint32_t n_capacity, int key_value) {
     (void)key_value;
     if (!ctx) return GMS_ERR_INVALID_ARG;
-    gms_status st = scratch_alloc(ctx->s, matrix_elems(n_capacity, 2));
+    gms_status st = scratch_alloc(ctx->s, matrix_elems(n_capacity, 2), true);
     if (st != GMS_SUCCESS) return st;
     ctx->capacity = n_capacity;
     ctx->allocated = 1;

@@ -87,12 +87,13 @@ struct Scratch {
     // Pinned host words that the kernels write the bucket starts of a call with
     // host results into (pinned_results).
     uint32_t* pin = nullptr;
+    bool host_results = false;  // holds a share in the device's pinned block
     int device = -1;
 };
 // Bucket counts up to which host results go through Scratch::pin.
 constexpr uint32_t kPinnedResults = 1024;
-// s.pin, a slot of the device's pinned block that the first call which needs it
-// takes and scratch_free gives back; NULL when none can be had.
+// s.pin, a slot of the device's pinned block (allocated with the scratch) that the first call
+// which needs it takes and scratch_free gives back; NULL when none can be had.
 uint32_t* pinned_results(Scratch& s);
 
 // Multisplits into more than 256 buckets run as a stable radix sort of the
@@ -120,7 +121,8 @@ gms_status run_large_multisplit(LargeScratch& L, Scratch& s, const uint32_t* kin
                                 uint32_t num_buckets, gms_bucket_desc d, uint32_t* d_offsets,
                                 hipStream_t stream);
 
-gms_status scratch_alloc(Scratch& s, size_t hist_elems);
+// host_results: the context's calls may want results on the host (pinned_results).
+gms_status scratch_alloc(Scratch& s, size_t hist_elems, bool host_results);
 void scratch_free(Scratch& s);
 // Matrix elements needed for n keys in B buckets (key-only and key-value tiles).
 size_t matrix_elems(uint32_t n, uint32_t num_buckets);

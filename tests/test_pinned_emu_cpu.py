@@ -54,3 +54,52 @@ def test_refused_pinned_memory_falls_back_to_the_copy(emu, refuse):  # noqa: F81
     kept = keys[keys < np.uint32(1 << 31)]
     assert count.value == kept.size
     np.testing.assert_array_equal(kout[:kept.size], kept)
+
+
+def test_calls_with_host_results_allocate_nothing(emu):  # noqa: F811
+    """Allocations belong to *_allocate: another thread may be capturing a graph
+    while a call runs."""
+    emu.gms_emu_alloc_calls.restype = ctypes.c_uint64
+    keys = W.uniform_keys(3000, seed=1)
+    for _ in range(2):
+        h = _multisplit_ctx(emu, 64, keys.size)
+        before = emu.gms_emu_alloc_calls()
+        for _ in range(2):
+            _host_starts(emu, h, keys, 64)
+        assert emu.gms_emu_alloc_calls() == before
+        emu.gms_multisplit_destroy(h)
+    kout, count = np.zeros_like(keys), ctypes.c_uint32(7)
+    h = ctypes.c_void_p()
+    assert emu.gms_compaction_create(ctypes.byref(h)) == 0
+    assert emu.gms_compaction_allocate(h, keys.size, 0) == 0
+    before = emu.gms_emu_alloc_calls()
+    assert emu.gms_compaction(h, p(keys), None, p(kout), None, keys.size, gms.delta_func(1 << 31).desc(),
+                              ctypes.addressof(count), None, None) == 0
+    assert emu.gms_emu_alloc_calls() == before
+    emu.gms_compaction_destroy(h)
+    assert count.value == np.count_nonzero(keys < np.uint32(1 << 31))
+
+
+def test_refused_pinned_memory_is_asked_for_once(emu, refuse):  # noqa: F811
+    """Calls do not ask again; a context allocated after the last one of the
+    device was released does, and contexts that outlive others keep their
+    results."""
+    emu.gms_emu_alloc_calls.restype = ctypes.c_uint64
+    keys = W.uniform_keys(3000, seed=5)
+    refuse(1)
+    h = _multisplit_ctx(emu, 64, keys.size)
+    before = emu.gms_emu_alloc_calls()
+    for _ in range(3):
+        _host_starts(emu, h, keys, 64)
+    assert emu.gms_emu_alloc_calls() == before
+    emu.gms_multisplit_destroy(h)
+    a, b = _multisplit_ctx(emu, 64, keys.size), _multisplit_ctx(emu, 8, keys.size)
+    _host_starts(emu, a, keys, 64)
+    _host_starts(emu, b, keys, 8)
+    assert emu.gms_multisplit_allocate(a, 2 * keys.size, 0) == 0  # anew: its slot goes back
+    _host_starts(emu, a, keys, 64)
+    emu.gms_multisplit_destroy(a)
+    _host_starts(emu, b, keys, 8)
+    emu.gms_multisplit_release(b)
+    emu.gms_multisplit_release(b)  # twice is harmless
+    emu.gms_multisplit_destroy(b)
