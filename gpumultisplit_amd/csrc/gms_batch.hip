@@ -256,13 +256,18 @@ gms_status BatchEngine::plan(const gms_batch_item* items, uint32_t count,
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-size_t BatchEngine::device_bytes() const {
-    const size_t m = std::max<uint64_t>(m_total, 4);
-    return align256(std::max<size_t>(num_instances, 1) * sizeof(BatchInst)) +
-           align256(std::max<size_t>(num_wide, 1) * sizeof(BatchWideInst)) +
-           align256(std::max<size_t>(num_work, 1) * sizeof(BatchWork)) + align256(m * 4) +
+size_t BatchEngine::table_bytes(size_t instances, size_t wide, size_t work, uint64_t matrix,
+                                size_t groups) {
+    const size_t m = std::max<uint64_t>(matrix, 4);
+    return align256(std::max<size_t>(instances, 1) * sizeof(BatchInst)) +
+           align256(std::max<size_t>(wide, 1) * sizeof(BatchWideInst)) +
+           align256(std::max<size_t>(work, 1) * sizeof(BatchWork)) + align256(m * 4) +
            align256(scan_partials_needed(m) * 4) + align256(scan_chunks(m) * sizeof(uint64_t)) +
-           align256(16 * std::max<size_t>(groups.size(), 1) * 4);
+           align256(16 * std::max<size_t>(groups, 1) * 4);
+}
+
+size_t BatchEngine::device_bytes() const {
+    return table_bytes(num_instances, num_wide, num_work, m_total, groups.size());
 }
 
 BatchDevice BatchEngine::carve(void* base) const {

@@ -92,6 +92,10 @@ class BatchEngine {
     // Device bytes the current plan needs, and its tables inside `base`
     // (256-byte aligned, device_bytes() long).
     size_t device_bytes() const;
+    // The same of a step with these counts.  The sum over several steps is at
+    // least that of the step which holds them all.
+    static size_t table_bytes(size_t instances, size_t wide, size_t work, uint64_t matrix,
+                              size_t groups);
     BatchDevice carve(void* base) const;
     // Copies the staged tables to the device on `stream` (asynchronous).
     gms_status upload(const BatchDevice& d, hipStream_t stream);

@@ -152,13 +152,22 @@ struct Req {
     }
 };
 
-// Device bytes one pass of n elements with 2^log_b matrix rows can need in a
-// step (its share of the step's tables; shares add up to at least the step).
-static size_t step_share(uint32_t n, int log_b, uint32_t tile_elems, size_t inst_bytes) {
-    const uint64_t tile = tile_elems;
-    const uint64_t tiles = n ? (n + tile - 1) / tile : 1;
+// Device bytes of a step that holds only one pass of n elements with 2^log_b
+// matrix rows: its share of a step's tables (shares add up to at least the step).
+static size_t step_share(uint32_t n, int log_b, uint32_t tile_elems, bool wide) {
+    const uint64_t tiles = n ? ((uint64_t)n + tile_elems - 1) / tile_elems : 1;
+    return BatchEngine::table_bytes(wide ? 0 : 1, wide ? 1 : 0, tiles,
+                                    ((uint64_t)1 << log_b) * tiles, 1);
+}
+
+// What a request must leave room for twice to be taken at all: its pass's own
+// tables, without the scan's status words (1/512 of the matrix) and the padding of empty
+// tables, which the budget's slack for fragmentation (1/16 of the arena) holds.
+static size_t least_share(uint32_t n, int log_b, uint32_t tile_elems, bool wide) {
+    const uint64_t tiles = n ? ((uint64_t)n + tile_elems - 1) / tile_elems : 1;
     const uint64_t m = ((uint64_t)1 << log_b) * tiles;
-    return round256(inst_bytes) + round256(tiles * sizeof(BatchWork)) + round256(m * 4) +
+    return round256(wide ? sizeof(BatchWideInst) : sizeof(BatchInst)) +
+           round256(tiles * sizeof(BatchWork)) + round256(m * 4) +
            round256(((m + kScanChunk - 1) / kScanChunk + 1) * 4) + 256;
 }
 
@@ -472,7 +481,11 @@ gms_status gms_server_submit(gms_server* s, const gms_request* q, uint64_t* tick
     const uint32_t K = s->cfg.items_per_thread;
     // tables of one pass: the 32-bit batched tile, or the 64-bit one
     const uint32_t tile = r->wide() ? wide_tile_elems(r->kw, r->vw) : kThreads * K;
-    const size_t inst = r->wide() ? sizeof(BatchWideInst) : sizeof(BatchInst);
+    size_t least = 0;
+    auto shares = [&](int log_b) {
+        least = r->tmp_bytes + 2 * least_share(q->n, log_b, tile, r->wide());
+        r->reserve = r->tmp_bytes + 2 * step_share(q->n, log_b, tile, r->wide());
+    };
     if (q->op == GMS_OP_MULTISPLIT) {
         gms_status st;
         if (r->wide()) {
@@ -484,22 +497,23 @@ gms_status gms_server_submit(gms_server* s, const gms_request* q, uint64_t* tick
         if (st != GMS_SUCCESS) return st;
         r->np = 1;
         const int lb = ceil_log2_u32(q->num_buckets);
-        r->reserve = 2 * step_share(q->n, lb < 1 ? 1 : lb, tile, inst);
+        shares(lb < 1 ? 1 : lb);
     } else if (q->op == GMS_OP_SORT) {
         r->np = wide_sort_passes(r->kw, q->digit_bits, r->pass);
         if (r->np == 0) return GMS_ERR_INVALID_ARG;
         r->tmp_bytes = round256(kb) + (kv ? round256(vb) : 0);
-        r->reserve = round256(r->tmp_bytes) + 2 * step_share(q->n, 8, tile, inst);
+        shares(8);
     } else {
         return GMS_ERR_INVALID_ARG;
     }
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->error != GMS_SUCCESS) return s->error;
     if (s->stopping) return GMS_ERR_INVALID_ARG;
-    if (r->reserve > s->budget()) {
+    if (least > s->budget()) {
         ++s->st.rejected;
         return GMS_ERR_CAPACITY;
     }
+    r->reserve = std::min(r->reserve, s->budget());
     r->ticket = s->next_ticket++;
     r->t_submit = Clock::now();
     s->by_ticket[r->ticket] = r;
@@ -537,6 +551,30 @@ gms_status gms_server_wait(gms_server* s, uint64_t ticket, double* latency_us) {
 }
 
 #ifdef GMS_HOST_EMULATION
+// Sum of the shares of multisplits of the given sizes into 2^log_b[i] buckets (32-bit, or
+// 64-bit pairs where wide[i]), and the bytes of the step that holds them all.
+gms_status gms_emu_step_bytes(const uint32_t* n, const uint32_t* log_b, const uint32_t* wide,
+                              uint32_t count, uint32_t items_per_thread, size_t* shares, size_t* step) {
+    static uint32_t dummy[8];  // planning touches no buffer
+    std::vector<gms_batch_item> items;
+    std::vector<BatchWideItem> wides;
+    *shares = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        const uint32_t B = 1u << log_b[i];
+        if (wide[i]) wides.push_back(BatchWideItem{dummy, dummy, dummy, dummy, n[i], B, 2, 2, {}, nullptr});
+        else items.push_back(gms_batch_item{dummy, nullptr, dummy, nullptr, n[i], B, {}, nullptr});
+        *shares += step_share(n[i], (int)log_b[i],
+                              wide[i] ? wide_tile_elems(2, 2) : (uint32_t)kThreads * items_per_thread,
+                              wide[i] != 0);
+    }
+    BatchEngine e;
+    e.tuning.items_per_thread = items_per_thread;
+    const gms_status st = e.plan(items.data(), (uint32_t)items.size(), wides.data(),
+                                 (uint32_t)wides.size(), 0);
+    *step = st == GMS_SUCCESS ? e.device_bytes() : 0;
+    e.release();
+    return st;
+}
 // Test hooks of the CPU emulation build only (not in the GPU library):
 // occupy or free a range of the server's arena, to test how steps are placed
 // in a fragmented arena.  The caller makes sure the server is idle.
