@@ -107,7 +107,6 @@ hipError_t two_shape(const ShortCall& c, const ShortPlan& p, uint32_t* H, const 
     switch (p.items) {
         case 4: return two_k<4, KW, VW>(c, p, H, f);
         case 8: return two_k<8, KW, VW>(c, p, H, f);
-        case 16: return two_k<16, KW, VW>(c, p, H, f);
         default: return hipErrorInvalidValue;
     }
 }
@@ -127,44 +126,62 @@ bool short_one_block(uint32_t n, uint32_t bits, uint32_t kw, uint32_t vw) {
     return n <= (bits > 8u && bits <= 12u ? 4096u : kw + vw > 3u ? 6144u : 8192u);
 }
 
-// Tiles of 4 elements per thread while that gives at most one tile per CU,
-// then 8 and 16, so that the call is one round of workgroups; a count
-// workgroup takes 4 tiles (C in gms_short.hpp) from the matrix size on where
-// every scatter workgroup's reading of all rows costs more than the longer
-// count kernel.  On MI355X (key-value, GPU us with items.group):
+// Tiles of 4 elements per thread while that gives at most one tile per CU, then
+// 8 (16 keep too few workgroups in flight: below); a count workgroup takes 4
+// tiles (C in gms_short.hpp) from the matrix size on where every scatter
+// workgroup's reading of all rows costs more than the longer count kernel.  On
+// MI355X (GPU us with items.group; key-value, uniform / sorted keys):
 //   256 buckets  60k keys 4.1 8.6, 4.4 9.0; 150k 4.1 11.4, 4.4 10.0;
-//                600k 8.1 18.6, 8.4 15.2; 1M 8.4 17.2, 16.4 19.1
-//   64 buckets   300k 8.1 9.8, 8.4 11.4; 1M 8.1 14.0, 8.4 13.6; 2M 16.1 20.0, 16.4 22.7
-// Against the three stages with their scan (the call's time before): 24.6 us
-// at 60k, 21.7 at 150k, 24.3 at 600k, 25.7 at 1M (256 buckets); 24.2 at 2M (64).
-// The upper ends are where the three stages are as fast: 2^21 keys up to 64
-// buckets (8 buckets 15.7 against 20.2 us there, 2 buckets key-only at 2^22
-// 24.4 against 21.2), 1.5 * 2^20 for 128 and 256 (2M: 27.0 against 26.7), 2^20
-// above (28.2 against 31.5 at 1024) and for 64-bit elements (64-bit keys with
-// 32-bit values, 256 buckets: 16.9 against 18.9 there, 21.7 against 21.0 at 1.5M).
-ShortPlan short_plan(uint32_t n, uint32_t num_buckets, uint32_t kw, uint32_t vw) {
-    const int cl = ceil_log2_u32(num_buckets);
-    const uint32_t lb = cl < 2 ? 2u : (uint32_t)cl;
-    ShortPlan p{0u, 1u, lb, 0u};
-    const bool wide = kw == 2 || vw == 2;
-    if (lb > (wide ? 8u : 10u)) return p;
-    const uint32_t top = wide || lb > 8 ? 1u << 20 : lb > 6 ? 3u << 19 : 1u << 21;
-    if (n > top) return p;
-    p.items = n <= (1u << 18) ? 4u : n <= (1u << 20) ? 8u : 16u;
+//                600k 8.1 18.6, 8.4 15.2; 1.1M 8.1 27.8 / 28.6, 8.4 17.1 / 19.2, 16.4 18.7 / 25.5
+//   64 buckets   300k 8.1 9.8, 8.4 11.4; 1.1M 8.1 15.9 / 17.7, 8.4 13.5 / 15.5, 16.1 16.1 / 22.2;
+//                2M 8.1 24.0 / 25.5, 8.4 16.9 / 19.4, 16.4 18.7 / 25.0
+//   2 buckets    1.1M 8.1 11.6 / 11.8, 16.1 12.8 / 14.7; 2M 8.1 14.7 / 15.1, 16.1 14.4 / 17.0
+static ShortPlan short_shape(uint32_t n, uint32_t log_b) {
+    ShortPlan p{n <= (1u << 18) ? 4u : 8u, 1u, log_b, 0u};
     const size_t tile = (size_t)kThreads * p.items;
     const size_t nt = ((size_t)n + tile - 1) / tile;
-    if ((nt << lb) > (p.items == 16u ? 48u * 1024u : 20u * 1024u)) p.group = 4u;
-    p.matrix_words = (nt + (p.group > 1u ? (nt + p.group - 1u) / p.group : 0u)) << lb;
+    if ((nt << log_b) > (p.items == 8u ? 16u * 1024u : 20u * 1024u)) p.group = 4u;
+    p.matrix_words = (nt + (p.group > 1u ? (nt + p.group - 1u) / p.group : 0u)) << log_b;
     return p;
 }
 
+// The largest short call: where the three stages are as fast.  Key-value,
+// uniform / sorted keys, three stages against this: 64 buckets 1.1M 19.0 / 20.8
+// and 13.5 / 15.5, 2M 21.0 / 24.8 and 16.9 / 19.4; 2 buckets 2M 15.0 / 15.9 and 14.7 / 15.1;
+// 256 buckets 1.3M 22.6 / 25.2 and 18.3 / 19.9, 1.53M 19.5 / 21.4 and 19.6 / 21.0, 2M 23.2 /
+// 26.7 and 25.5 / 26.6; 1024 buckets 1M 31.5 and 28.2; 64-bit keys with 32-bit
+// values, 256 buckets, 1M 18.9 and 16.9, 1.5M 21.0 and 21.7.
+static uint32_t short_top(uint32_t log_b, bool wide) {
+    return wide || log_b > 8 ? 1u << 20 : log_b > 6 ? 3u << 19 : 1u << 21;
+}
+
+// A whole number of the three stages' tiles has no ragged workgroup, whose
+// guarded loads set the time of a call this short: 3 * 2^19 key-value elements
+// into 256 buckets take them 16.6 us (1.53M: 19.5) and the two launches 19.4;
+// 2 buckets 11.4 and 12.2; 3 * 2^18 into 1024 buckets 21.0 and 24.6.  With 16 to
+// 64 buckets the two launches stay ahead (64 buckets 15.3 and 14.2).
+static bool whole_tiles_win(uint32_t n, uint32_t log_b) {
+    if (n % (uint32_t)(kThreads * tune_items(1, false, false)) != 0) return false;
+    return log_b == 10 ? n >= 3u << 18 : (log_b <= 3 || log_b >= 7) && n > 1u << 20;
+}
+
+ShortPlan short_plan(uint32_t n, uint32_t num_buckets, uint32_t kw, uint32_t vw) {
+    const int cl = ceil_log2_u32(num_buckets);
+    const uint32_t lb = cl < 2 ? 2u : (uint32_t)cl;
+    const bool wide = kw == 2 || vw == 2;
+    if (lb > (wide ? 8u : 10u) || n > short_top(lb, wide) || (!wide && whole_tiles_win(n, lb)))
+        return ShortPlan{0u, 1u, lb, 0u};
+    return short_shape(n, lb);
+}
+
 size_t short_matrix_words(uint32_t n_capacity, uint32_t num_buckets) {
+    const int cl = ceil_log2_u32(num_buckets);
+    const uint32_t lb = cl < 2 ? 2u : (uint32_t)cl;
+    if (lb > 10u) return 0;
     // The largest at the ends of the ranges of one tile length.
     size_t m = 0;
-    for (uint32_t end : {1u << 18, 1u << 20, 3u << 19, 1u << 21}) {
-        const uint32_t n = n_capacity < end ? n_capacity : end;
-        m = std::max(m, short_plan(n, num_buckets, 1, 1).matrix_words);
-    }
+    for (uint32_t end : {1u << 18, short_top(lb, false)})
+        m = std::max(m, short_shape(n_capacity < end ? n_capacity : end, lb).matrix_words);
     return m;
 }
 
@@ -215,3 +232,18 @@ hipError_t launch_short_two(const ShortCall& c, const ShortPlan& p, uint32_t* H,
 }
 
 }  // namespace gms
+
+#ifdef GMS_HOST_EMULATION
+// Test hook of the CPU emulation build only: the plan of a call, and the matrix
+// words of a context for up to n_capacity elements.
+extern "C" void gms_emu_short_plan(uint32_t n, uint32_t num_buckets, uint32_t kw, uint32_t vw,
+                                   uint32_t* items, uint32_t* group, uint64_t* words) {
+    const gms::ShortPlan p = gms::short_plan(n, num_buckets, kw, vw);
+    *items = p.items;
+    *group = p.group;
+    *words = p.matrix_words;
+}
+extern "C" uint64_t gms_emu_matrix_words(uint32_t n_capacity, uint32_t num_buckets) {
+    return gms::matrix_elems(n_capacity, num_buckets);
+}
+#endif
