@@ -349,11 +349,12 @@ gms_status run_prescan_only(Scratch& s, const uint32_t* kin, uint32_t n, uint32_
 
 // The multisplit: one or two launches for short inputs (identifier `any`),
 // else prescan -> scan -> postscan with the identifier that `with_f` hands to
-// its callback (the built-in kinds by descriptor, or a given functor).
+// its callback (the built-in kinds by descriptor, or a given functor).  pass: one
+// digit pass of several.
 template <class WithF>
 static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
                              uint32_t* vout, uint32_t n, uint32_t B, uint32_t* d_offsets,
-                             hipStream_t stream, Profiler* prof, const DigitOfF& any,
+                             hipStream_t stream, Profiler* prof, const DigitOfF& any, bool pass,
                              WithF&& with_f) {
     const bool kv = vin != nullptr;
     if (n == 0) return d_offsets ? hip_status(launch_fill(d_offsets, 0u, B, stream)) : GMS_SUCCESS;
@@ -377,7 +378,7 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
     MsCall c;
     gms_status st = plan_call(s, kin, vin, kout, vout, n, B, kv, stream, c);
     if (st != GMS_SUCCESS) return st;
-    c.reg_rank = reg_rank(c.log_b, kv, n, d_offsets && apart);
+    c.reg_rank = reg_rank(c.log_b, kv, n, d_offsets && apart, pass);
     if (c.reg_rank && apart) {
         c.offs = d_offsets;
         c.nb = B;
@@ -401,14 +402,14 @@ gms_status run_multisplit(Scratch& s, const uint32_t* kin, const uint32_t* vin, 
                           uint32_t* vout, uint32_t n, uint32_t B, gms_bucket_desc d,
                           uint32_t* d_offsets, hipStream_t stream, Profiler* prof) {
     return run_stages(s, kin, vin, kout, vout, n, B, d_offsets, stream, prof,
-                      DigitOfF{AnyF::make(d.kind, d.param, d.width, B), 0u, ~0u},
+                      DigitOfF{AnyF::make(d.kind, d.param, d.width, B), 0u, ~0u}, false,
                       [&](auto&& launch) { return with_functor(B, d, launch); });
 }
 
 gms_status run_multisplit_digit(Scratch& s, const uint32_t* kin, const uint32_t* vin,
                                 uint32_t* kout, uint32_t* vout, uint32_t n, uint32_t B,
                                 const DigitOfF& f, hipStream_t stream) {
-    return run_stages(s, kin, vin, kout, vout, n, B, nullptr, stream, nullptr, f,
+    return run_stages(s, kin, vin, kout, vout, n, B, nullptr, stream, nullptr, f, true,
                       [&](auto&& launch) { return launch(f); });
 }
 
@@ -1322,3 +1323,10 @@ gms_status gms_copy_u32(const uint32_t* src, uint32_t* dst, size_t n, void* stre
 }
 
 }  // extern "C"
+
+#ifdef GMS_HOST_EMULATION
+// Test hook of the CPU emulation build only: the postscan's form.
+extern "C" int gms_emu_reg_rank(int log_b, int kv, uint32_t n, int starts, int pass) {
+    return gms::reg_rank(log_b, kv != 0, n, starts != 0, pass != 0);
+}
+#endif

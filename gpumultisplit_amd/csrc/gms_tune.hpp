@@ -69,40 +69,51 @@ constexpr bool tune_alias(int log_b, int items, bool kv, int level_bits) {
     return kv && cnt_row(1 << level_bits) <= items && !(log_b >= 7 && items < 28);
 }
 
-// Keys from which a class always loads a postscan tile through LDS and ranks it
-// with register counters (ms_postscan_reg_kernel) instead of blocked loads and
-// LDS counters; 0: no such size.  On MI355X, whole call, LDS counters against
-// registers (us):
-//   key-value  2 buckets 10M 48.7 / 47.0, 13M 60.3 / 55.9, 2^24 73.1 / 68.9, 2^25
-//              134 / 132, 2^26 240 / 238; 16 buckets 13M 66.6 / 62.0, 2^25 139 / 134,
-//              2^26 257 / 238, 90M 347 / 336; 32 buckets 20M 86.7 / 90.6, 2^26 258 / 243
-//   key-only   2 buckets 10M 29.1 / 27.5, 13M 35.7 / 32.6, 2^25 85.2 / 84.2, 2^26 143 /
-//              140; 8 buckets 13M 36.6 / 34.1, 2^26 144 / 137
-// At 3M to 8M keys both are the same or the LDS counters up to 5 % faster.  With
-// more buckets it depends on the identifier and on what wrote the input: 2^25 pairs
-// in 256 buckets 157 / 149 by range but 153 / 154 by division, passes of an 8-bit
-// sort of 2^25 keys 98 / 107, of 2^26 pairs 277 / 413.
+// Few buckets: the classes whose postscan loads its tile through LDS and ranks it with
+// register counters (ms_postscan_reg_kernel), instead of blocked loads and LDS
+// counters, whenever the call wants the bucket starts, and from some size on without.
+constexpr bool reg_rank_few(int log_b, bool kv) { return log_b <= (kv ? 4 : 3); }
+
+// Keys from which a class takes it in every call; 0: no such size.  On MI355X, whole
+// call without starts, registers / LDS counters, the worst of uniform, sorted and
+// one-key-in-ten keys and of range, division and digit identifiers, then the best:
+//   key-value  2 buckets 9.5M 1.00 .98, 2^24 .96 .95, 50M 1.02 .99, 2^26 .96 .94; 8 buckets
+//              9.5M 1.04 1.00, 13.5M 1.03 1.00, 2^24 .98 .94, 2^25 .98 .94, 2^26 .96 .89; 16
+//              buckets 9.5M 1.08 1.04, 15M 1.05 1.00, 20M 1.05 .98, 2^25 1.00 .96, 2^26 .93 .89
+//   key-only   2 buckets 13.5M 1.03 .97, 2^25 1.00 .98, 2^26 .85 .82; 4 buckets 9.5M 1.06
+//              1.02, 13.5M 1.07 .99, 20M 1.04 .99, 2^26 .88 .84; 8 buckets 13.5M 1.06 .99, 50M
+//              1.04 1.00, 2^26 .94 .87
+// With 32 buckets of pairs at 2^26 uniform keys gain (258 / 243 us) what sorted ones
+// lose (256 / 281); with more it depends on the identifier and on what wrote the
+// input: 2^25 pairs in 256 buckets 157 / 149 by range but 153 / 154 by division,
+// passes of an 8-bit sort of 2^25 keys 98 / 107, of 2^26 pairs 277 / 413.
 constexpr uint32_t reg_rank_from(int log_b, bool kv) {
-    return log_b <= (kv ? 4 : 3) ? 9u << 20 : (kv && log_b == 5 ? kLongTileMin : 0u);
+    if (!reg_rank_few(log_b, kv)) return 0u;
+    return kv ? (log_b <= 3 ? 1u << 24 : 1u << 25) : 1u << 26;
 }
 
-// Keys below which it does so in a call that wants the bucket starts: this form
+// Keys below which a class takes it in a call that wants the bucket starts: this form
 // writes them, the other leaves them to a launch of about 4 us and the gap before
-// it.  Range / division / digit identifier, as above:
-//   key-only   16 buckets 2.2M 19.9 / 18.2, 21.8 / 20.1, 20.8 / 18.7; 64 buckets 6M
-//              27.2 / 23.5, 29.5 / 26.1, 27.4 / 24.9, at 9.5M 35.9 / 32.6, 39.2 / 37.5,
-//              36.5 / 35.8, at 24M by digit 63 / 68; 256 buckets 4M 27.8 / 23.3, 29.6 /
-//              25.9, 28.4 / 25.0
-//   key-value  2 buckets 4M 24.9 / 18.9 by range, 8M 32.8 / 31.2; 16 buckets 6M 35.6 /
-//              34.2, 36.0 / 35.1, 35.5 / 34.0; 64 buckets 6M 34.5 / 32.7, 36.0 / 34.9,
-//              34.7 / 33.0, at 9.5M 44.1 / 45.3, 46.8 / 48.8, 45.1 / 45.4; 256 buckets 6M
-//              42.4 / 37.0, 43.9 / 38.9, 42.9 / 36.6
+// it.  As above (the other form with its launch):
+//   key-value  2 buckets 2.3M .87 .84, 9.5M .96 .94, 2^25 .97 .96; 16 buckets 4.2M 1.01 .99, 6.3M
+//              1.04 1.00, 9.5M 1.04 .99, 2^24 .98 .94; 64 buckets 4.2M .98 .96, 6.3M 1.03 .98, 8.5M
+//              1.02 .97; 256 buckets 4.2M .88 .83, 6.3M 1.00 .93; at 9.5M 64 buckets 44.1 / 45.3 us
+//              by range, 46.8 / 48.8 by division
+//   key-only   2 buckets 6.3M .92 .87; 8 buckets 6.3M .95 .92, 50M 1.01 .97; 64 buckets 6.3M .98
+//              .93, 8.5M .97 .89, at 24M by digit 63 / 68 us; 256 buckets 4.2M .88 .84, 8.5M .96 .90
 constexpr uint32_t reg_rank_starts_below(int log_b, bool kv) {
-    return log_b > 8 ? 0u : (kv && log_b > 3 ? 7u << 20 : 9u << 20);
+    if (reg_rank_few(log_b, kv)) return 0xFFFFFFFFu;
+    return log_b > 8 ? 0u : (kv ? 7u << 20 : 9u << 20);
 }
 
-constexpr bool reg_rank(int log_b, bool kv, uint32_t n, bool starts) {
+// The form of one call; `pass`: of one digit pass of a sort or of a multisplit into
+// many buckets.  Those read what a kernel has just written: pairs gain only where the
+// loads stream (4-bit sort of 2^26 2030 / 1817 us, 5-bit 1803 / 1664, of 2^25 1021 / 988;
+// but 2^25 sorted pairs into 500,000 buckets, last pass 3 bits, 478 / 490), key-only
+// ones lose (2048 buckets, last pass 3 bits: 2^25 keys 199 / 203, 2^26 368 / 377).
+constexpr bool reg_rank(int log_b, bool kv, uint32_t n, bool starts, bool pass) {
     const uint32_t from = reg_rank_from(log_b, kv);
+    if (pass) return kv && from && n >= kStreamLoadMin;
     return (from && n >= from) || (starts && n < reg_rank_starts_below(log_b, kv));
 }
 
