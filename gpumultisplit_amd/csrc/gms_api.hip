@@ -66,12 +66,8 @@ static size_t stage_matrix_elems(uint32_t n, uint32_t num_buckets) {
         // 64-bit elements take passes of at most 256 buckets; 32-bit ones up to
         // kSinglePassBuckets one pass, above it passes of at most 512.
         size_t m = stage_matrix_elems(n, 256);
-        uint32_t width[3] = {0, 0, 0};
         int lb = ceil_log2_u32(num_buckets);
-        if (num_buckets > kSinglePassBuckets) {
-            (void)large_passes((uint32_t)lb, true, false, width);
-            lb = (int)width[0];  // the widest; key-only passes are the same or of 8 bits
-        }
+        if (num_buckets > kSinglePassBuckets) lb = lb == 17 || lb == 18 ? 9 : 8;  // large_passes
         if (lb > 8) {
             const uint32_t tko = std::min(tile_keys(lb, false, 0), tile_keys(lb, false, kLongTileMin));
             const uint32_t tkv = std::min(tile_keys(lb, true, 0), tile_keys(lb, true, kLongTileMin));

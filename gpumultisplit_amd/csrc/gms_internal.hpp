@@ -100,10 +100,10 @@ uint32_t* pinned_results(Scratch& s);
 // bucket ids (gms_large.hip); up to this many buckets.
 constexpr uint32_t kMaxBuckets = 1u << 20;
 
-// Widths, at most 9 bits, of the LSD passes over a bits-bit id (11 to 20 bits; 9 to 20 with
-// 64-bit elements, whose passes take at most 8 bits), least significant first;
-// returns their number.
-int large_passes(uint32_t bits, bool kv, bool wide, uint32_t (&width)[3]);
+// Widths of the LSD passes of an n-element call over a bits-bit id (11 to 20 bits; 9 to
+// 20 with 64-bit elements), least significant first; returns their number.  At most 9
+// bits with ids of 17 and 18 bits of 32-bit elements, else at most 8.
+int large_passes(uint32_t bits, bool kv, bool wide, uint32_t n, uint32_t (&width)[3]);
 
 struct LargeScratch {
     uint32_t* ktmp = nullptr;  // keys between passes

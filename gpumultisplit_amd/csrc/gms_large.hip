@@ -42,18 +42,39 @@ void large_scratch_free(LargeScratch& L) {
     L.cap = 0;
 }
 
-// Passes of equal width where that pays, else 8 bits a pass.  On MI355X, whole
-// call in us, 8 bits a pass against the rule, key-value / key-only:
-//   13 bits  4M 64.4 / 59.5 -> 61.1 / 55.3 (7 + 6), 2^27 1101 / 749 -> 1063 / 743
-//   17 bits  4M 86.6 / 78.9 -> 73.8 / 64.5 (9 + 8), 2^27 1629 / 1091 -> 1244 / 961
-//   18 bits  4M 87.5 / 80.3 -> 79.4 / 77.4 (9 + 9), 2^27 1633 / 1095 -> 1352 / 1013
-//   20 bits  4M 94.1 -> 89.7 (7 + 7 + 6), 2^27 1657 -> 1596; key-only 207 -> 213 at 20M,
-//            so key-only keeps 8 + 8 + 4
-//   11 bits  8 + 3: 4M 56.3 / 50.8, 20M 184 / 129 (6 + 5: 60.0 / 55.2, 183 / 140)
-// 64-bit elements keep 8 bits a pass.
-int large_passes(uint32_t bits, bool kv, bool wide, uint32_t (&width)[3]) {
-    const uint32_t np = bits <= (wide ? 16u : 18u) ? 2u : 3u;
-    const bool even = !wide && bits > 11u && (np == 2u || kv);
+// Passes of equal width where no key distribution measured slower, else 8 bits
+// a pass.  On MI355X, time over that of 8 bits a pass, uniform / sorted / nine in ten
+// keys equal:
+//   12 bits  6 + 6: 1.6M .91 / .83 / .84; 9M key-only .99 / 1.07 / 1.07, key-value .94 /
+//            1.05 / 1.03; 2^25 key-value .96 / 1.01 / 1.00, 50M .94 / .95 / .98
+//   13 bits  7 + 6: 1.1M .96 / .96 / .96, 3M .91 / .97 / .97, 2^24 .98 / 1.00 / 1.00
+//   14 bits  7 + 7: 1.9M 1.18 / 1.26 / 1.23, 2^27 key-only 1.08 / 1.07 / 1.04, key-value .95 /
+//            1.10 / 1.04
+//   17 bits  9 + 8: 1M .85 / .85 / .88, 9M .84 / .85 / .85, 2^27 key-value .77 / .81 / .81,
+//            key-only .88 / 1.10 / 1.00 but 6 + 6 + 5 .95 / 1.00 / .97
+//   18 bits  9 + 9: 1M .91 / .91 / .99, 9M .91 / .94 / .93, 2^27 key-value .83 / .90 / .91,
+//            key-only .99 / 1.34 / 1.30 but 6 + 6 + 6 .95 / 1.03 / 1.00; 1.3M 1.05 / 1.06 / 1.23,
+//            where 8-bit passes still take two launches and 9-bit ones do not
+//   19 bits  7 + 6 + 6, key-value: 1.9M .93 / .93 / .94, 3M 1.03 / 1.02 / 1.05, 2^24 .96 / 1.01 / 1.02
+//   20 bits  7 + 7 + 6, key-value: 1.3M .96 / .96 / .97, 1.9M 1.04 / 1.03 / 1.04, 9M 1.01 / 1.01 / 1.06
+// 11 bits stay 8 + 3 (6 + 5: 9M 1.04 / 1.10 / 1.09), 64-bit elements at 8 bits a pass.
+int large_passes(uint32_t bits, bool kv, bool wide, uint32_t n, uint32_t (&width)[3]) {
+    uint32_t np = bits <= (wide ? 16u : 18u) ? 2u : 3u;
+    bool even = false;
+    if (!wide) {
+        switch (bits) {
+            case 12: even = n <= 1u << 21 || (kv && n >= 1u << 25); break;
+            case 13: even = true; break;
+            case 17:
+            case 18:
+                even = !(bits == 18 && n > 1u << 20 && n <= 3u << 19);
+                if (!even || (!kv && n >= kLongTileMin)) np = 3;
+                break;
+            case 19: even = kv && n <= 1u << 21; break;
+            case 20: even = kv && n <= 3u << 19; break;
+            default: break;
+        }
+    }
     for (uint32_t i = 0, left = bits; i < np; ++i) {
         width[i] = even ? (left + (np - i) - 1u) / (np - i) : (left < 8u ? left : 8u);
         left -= width[i];
@@ -80,7 +101,7 @@ gms_status run_large_multisplit(LargeScratch& L, Scratch& s, const uint32_t* kin
         return hip_status(launch_bucket_starts<1>(kout, n, B, base, d_offsets, stream));
     }
     uint32_t width[3], shift = 0;
-    const int passes = large_passes((uint32_t)bits, kv, false, width);
+    const int passes = large_passes((uint32_t)bits, kv, false, n, width);
     const uint32_t* sk = kin;
     const uint32_t* sv = vin;
     for (int p = 0; p < passes; shift += width[p++]) {
@@ -99,3 +120,13 @@ gms_status run_large_multisplit(LargeScratch& L, Scratch& s, const uint32_t* kin
 }
 
 }  // namespace gms
+
+#ifdef GMS_HOST_EMULATION
+// Test hook of the CPU emulation build only: the passes of a call.
+extern "C" int gms_emu_large_passes(uint32_t bits, int kv, int wide, uint32_t n, uint32_t* width) {
+    uint32_t w[3] = {0, 0, 0};
+    const int np = gms::large_passes(bits, kv != 0, wide != 0, n, w);
+    for (int i = 0; i < 3; ++i) width[i] = w[i];
+    return np;
+}
+#endif

@@ -119,7 +119,7 @@ constexpr bool reg_rank(int log_b, bool kv, uint32_t n, bool starts, bool pass) 
 
 // Bucket counts up to this run in one prescan/scan/postscan pass (three LDS
 // ranking passes of at most 4 bits above 256); more take LSD passes over
-// 8-bit digits of the bucket id.
+// digits of the bucket id (large_passes).
 constexpr uint32_t kSinglePassBuckets = 1024;
 
 // Keys per tile for an input of n keys.  The shortest tile, used to size the

@@ -139,7 +139,7 @@ gms_status run_wide_large(Scratch& s, uint32_t* ktmp, uint32_t* vtmp, const uint
         return wide_starts(kout, n, kw, B, d, d_offsets, stream);
     }
     uint32_t width[3], shift = 0;
-    const int passes = large_passes((uint32_t)bits, vw != 0, true, width);
+    const int passes = large_passes((uint32_t)bits, vw != 0, true, n, width);
     const uint32_t* sk = kin;
     const uint32_t* sv = vin;
     for (int p = 0; p < passes; shift += width[p++]) {
