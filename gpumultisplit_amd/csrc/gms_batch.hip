@@ -121,13 +121,25 @@ gms_status BatchEngine::reserve_tables(uint32_t instances, uint64_t work_items) 
 
 // Tile shape of a step that was not tuned.  Steps of few keys are bound by the
 // latency of a tile and by their ragged tiles, large ones by bandwidth, where
-// longer output runs pay.  On MI355X (us a run at 8 / 16 / 24 keys per thread):
-// 64 buckets 1.1M pairs 17 / 23 / 25, 11M 48 / 56 / 62, 72M 355 / 303 / 301; 256
-// buckets 11M 61 / 64 / 66; sorts and multisplits of 36M pairs 361 / 344 / 359.
+// longer output runs pay: from 2^24 keys on into more than 128 buckets, from 2^26
+// on into fewer, but not key-only ones into up to 32.  On MI355X (us a run at 8 /
+// 16 / 24 keys per thread):
+//   64 buckets   pairs 11M 48 / 56 / 61, 43M 198 / 187 / 195, 72M 346 / 310 / 303; keys 43M 125 / 120 / 121
+//   256 buckets  pairs 11M 60 / 63 / 66, 21M 142 / 116 / 115, 43M 301 / 225 / 214; keys 11M 53 / 52 / 52,
+//                21M 90 / 83 / 81, 43M 176 / 151 / 143
+//   128 buckets  pairs 21M 112 / 104 / 109, 43M 230 / 201 / 201; keys 43M 143 / 133 / 132
+//   32 buckets   keys 72M 190 / 187 / 199, 117M 302 / 297 / 313; 8 buckets keys 117M 258 / 255 / 261
+// A step has one shape: that of the larger part of its keys.
 static uint32_t default_items(const gms_batch_item* items, uint32_t count) {
-    uint64_t keys = 0;
-    for (uint32_t i = 0; i < count; ++i) keys += items[i].n;
-    return keys < (1u << 24) ? 8u : keys < (1u << 26) ? 16u : 24u;
+    uint64_t keys = 0, many = 0, few_ko = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        keys += items[i].n;
+        if (items[i].num_buckets > 128u) many += items[i].n;
+        if (items[i].num_buckets <= 32u && !items[i].d_value_in) few_ko += items[i].n;
+    }
+    if (keys < (1u << 24)) return 8u;
+    if (keys < (1u << 26)) return 2u * many >= keys ? 24u : 16u;
+    return 2u * few_ko > keys ? 16u : 24u;
 }
 
 gms_status BatchEngine::plan(const gms_batch_item* items, uint32_t count,
@@ -317,11 +329,12 @@ uint32_t BatchEngine::grid_for(const BatchGroup& g, bool post) const {
     const uint32_t nw = g.w1 - g.w0;
     if (!tuning.persistent) return nw;
     int occ = 1;
+    const uint32_t keys = (uint32_t)keys_total;
     switch (items_) {
-        case 8: occ = batch_occupancy_k8(g.log_b, g.kv, post); break;
-        case 16: occ = batch_occupancy_k16(g.log_b, g.kv, post); break;
-        case 24: occ = batch_occupancy_k24(g.log_b, g.kv, post); break;
-        default: occ = batch_occupancy_k32(g.log_b, g.kv, post); break;
+        case 8: occ = batch_occupancy_k8(g.log_b, g.kv, post, keys); break;
+        case 16: occ = batch_occupancy_k16(g.log_b, g.kv, post, keys); break;
+        case 24: occ = batch_occupancy_k24(g.log_b, g.kv, post, keys); break;
+        default: occ = batch_occupancy_k32(g.log_b, g.kv, post, keys); break;
     }
     // At least 8 workgroups (one per XCD) whenever there are 8 items, so that
     // every XCD's range of items has a workgroup to drain it.

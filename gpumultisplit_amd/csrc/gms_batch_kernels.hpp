@@ -14,6 +14,8 @@
 // obase_i + n_i, which closes its last bucket run.
 #pragma once
 
+#include <type_traits>
+
 #include "gms_kernels.hpp"
 #include "gms_rank.hpp"
 
@@ -147,9 +149,27 @@ __global__ __launch_bounds__(kThreads) void ms_batch_prescan_kernel(
     }
 }
 
-// Tiles of 32 keys per thread rank with LDS counters (postscan_rank): register
-// counters would leave one workgroup per CU (11M pairs into 64 buckets 91 to
-// 115 us, against 82).
+// Keys of a step from which tiles of K keys per thread rank with LDS counters
+// (postscan_rank); kNoLds: never.  Steps of few keys are bound by the latency of a
+// tile, where register counters win; large ones by bandwidth.  On MI355X, us a
+// run, registers / LDS counters:
+//   K = 32 always: register counters would leave one workgroup per CU (11M pairs
+//     into 64 buckets 91 to 115, against 82)
+//   K = 24 key-only: 32 buckets 42M 121 / 121, 72M 199 / 189; 64 buckets 26M 80 / 82, 72M 201 /
+//     193, 117M 323 / 311; 256 buckets 26M 94 / 99, 43M 143 / 142, 72M 241 / 231, 117M 388 / 378;
+//     16 buckets 72M 177 / 177; pairs 256 buckets 72M 338 / 355
+//   K = 16 key-only: 64 buckets 72M 199 / 196, 117M 317 / 312; 256 buckets 72M 259 / 245; 32 buckets
+//     72M 187 / 192
+//   K = 8 pairs: 64 buckets 21M 96 / 98, 26M 118 / 113, 43M 198 / 184; 256 buckets 26M 184 / 175, 72M 518 /
+//     487; 8 buckets 43M 165 / 164, 117M 451 / 436
+constexpr uint32_t kNoLds = 0xFFFFFFFFu;
+constexpr uint32_t batch_lds_from(int log_b, int items, bool kv) {
+    if (items >= 32) return 0u;
+    if (items == 24) return !kv && log_b >= 5 ? 1u << 26 : kNoLds;
+    if (items == 16) return !kv && log_b >= 6 ? 1u << 26 : kNoLds;
+    return kv && log_b >= 3 ? 3u << 23 : kNoLds;
+}
+
 template <int LOG_B, int K, int LEVEL_BITS, bool KV, bool VEC, bool ALIAS>
 __device__ __forceinline__ void batch_postscan_item_lds(
     const BatchInst* __restrict__ inst, const BatchWork* __restrict__ work, uint32_t w,
@@ -212,9 +232,7 @@ struct BatchSmem {
     uint32_t bs[kWaves];
 };
 
-// Ranked with register counters (gms_rank.hpp), as the short-input kernels: a
-// step's tiles are mostly few and ragged, and what bounds them is the latency
-// of one tile.
+// Ranked with register counters (gms_rank.hpp), as the short-input kernels.
 template <int LOG_B, int K, bool KV, bool VEC>
 __device__ __forceinline__ void batch_postscan_item(const BatchInst* __restrict__ inst,
                                                     const BatchWork* __restrict__ work, uint32_t w,
@@ -266,7 +284,7 @@ __device__ __forceinline__ void batch_postscan_item(const BatchInst* __restrict_
     }
 }
 
-template <int LOG_B, int K, bool KV, bool VEC, bool PERSIST>
+template <int LOG_B, int K, bool KV, bool VEC, bool PERSIST, bool LDS>
 __global__ __launch_bounds__(kThreads) void ms_batch_postscan_kernel(
     const BatchInst* __restrict__ inst, const BatchWork* __restrict__ work, uint32_t num_work,
     const uint32_t* __restrict__ G, uint32_t m_total, uint32_t keys_total,
@@ -281,7 +299,7 @@ __global__ __launch_bounds__(kThreads) void ms_batch_postscan_kernel(
                 item(R.begin + i);
         }
     };
-    if constexpr (K < 32) {
+    if constexpr (!LDS) {
         __shared__ __attribute__((aligned(16))) BatchSmem<LOG_B, K, KV> sm;
         each([&](uint32_t w) {
             batch_postscan_item<LOG_B, K, KV, VEC>(inst, work, w, G, m_total, keys_total, sm);
@@ -334,11 +352,11 @@ hipError_t launch_batch_postscan_k8(const BatchLaunch& c);
 hipError_t launch_batch_postscan_k16(const BatchLaunch& c);
 hipError_t launch_batch_postscan_k24(const BatchLaunch& c);
 hipError_t launch_batch_postscan_k32(const BatchLaunch& c);
-// Resident workgroups per CU of the persistent batch kernels.
-int batch_occupancy_k8(int log_b, bool kv, bool postscan);
-int batch_occupancy_k16(int log_b, bool kv, bool postscan);
-int batch_occupancy_k24(int log_b, bool kv, bool postscan);
-int batch_occupancy_k32(int log_b, bool kv, bool postscan);
+// Resident workgroups per CU of the persistent batch kernels, for a step of `keys` keys.
+int batch_occupancy_k8(int log_b, bool kv, bool postscan, uint32_t keys);
+int batch_occupancy_k16(int log_b, bool kv, bool postscan, uint32_t keys);
+int batch_occupancy_k24(int log_b, bool kv, bool postscan, uint32_t keys);
+int batch_occupancy_k32(int log_b, bool kv, bool postscan, uint32_t keys);
 
 template <int K>
 struct BatchKernels {
@@ -358,26 +376,49 @@ struct BatchKernels {
         if (c.vec && c.stream_loads) return prescan_v<LOG_B, true, false, true>(c);
         return c.vec ? prescan_v<LOG_B, true, false>(c) : prescan_v<LOG_B, false, false>(c);
     }
-    template <int LOG_B, bool KV, bool VEC, bool P>
+    template <int LOG_B, bool KV, bool VEC, bool P, bool LDS>
     static hipError_t postscan_v(const BatchLaunch& c) {
-        hipLaunchKernelGGL((ms_batch_postscan_kernel<LOG_B, K, KV, VEC, P>), dim3(c.grid),
+        hipLaunchKernelGGL((ms_batch_postscan_kernel<LOG_B, K, KV, VEC, P, LDS>), dim3(c.grid),
                            dim3(kThreads), 0, c.stream, c.inst, c.work, c.num_work,
                            (const uint32_t*)c.H, c.m_total, c.keys_total, c.queue);
         return hipGetLastError();
     }
-    template <int LOG_B, bool KV>
-    static hipError_t postscan(const BatchLaunch& c) {
+    template <int LOG_B, bool KV, bool LDS>
+    static hipError_t postscan_l(const BatchLaunch& c) {
         if (c.persistent)
-            return c.vec ? postscan_v<LOG_B, KV, true, true>(c) : postscan_v<LOG_B, KV, false, true>(c);
-        return c.vec ? postscan_v<LOG_B, KV, true, false>(c) : postscan_v<LOG_B, KV, false, false>(c);
+            return c.vec ? postscan_v<LOG_B, KV, true, true, LDS>(c)
+                         : postscan_v<LOG_B, KV, false, true, LDS>(c);
+        return c.vec ? postscan_v<LOG_B, KV, true, false, LDS>(c)
+                     : postscan_v<LOG_B, KV, false, false, LDS>(c);
+    }
+    // Calls fn with whether a step of `keys` keys ranks with LDS counters.
+    template <int LOG_B, bool KV, class Fn>
+    static auto with_form(uint32_t keys, Fn&& fn) {
+        constexpr uint32_t from = batch_lds_from(LOG_B, K, KV);
+        if constexpr (from == 0) {
+            return fn(std::true_type{});
+        } else {
+            if constexpr (from != kNoLds)
+                if (keys >= from) return fn(std::true_type{});
+            return fn(std::false_type{});
+        }
     }
     template <int LOG_B, bool KV>
-    static int occupancy(bool post) {
+    static hipError_t postscan(const BatchLaunch& c) {
+        return with_form<LOG_B, KV>(c.keys_total, [&](auto lds) {
+            return postscan_l<LOG_B, KV, decltype(lds)::value>(c);
+        });
+    }
+    template <int LOG_B, bool KV>
+    static int occupancy(bool post, uint32_t keys) {
         int occ = 0;
         hipError_t e;
         if (post) {
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &occ, ms_batch_postscan_kernel<LOG_B, K, KV, true, true>, kThreads, 0);
+            e = with_form<LOG_B, KV>(keys, [&](auto lds) {
+                return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                    &occ, ms_batch_postscan_kernel<LOG_B, K, KV, true, true, decltype(lds)::value>,
+                    kThreads, 0);
+            });
         } else {
             e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &occ, ms_batch_prescan_kernel<LOG_B, K, true, true>, kThreads, 0);
@@ -425,8 +466,8 @@ struct BatchKernels {
         GMS_BATCH_SWITCH(BatchKernels<KK>::postscan, (c), c.log_b, c.kv)                      \
         return hipErrorInvalidValue;                                                     \
     }                                                                                    \
-    int batch_occupancy_k##KK(int log_b, bool kv, bool post) {                           \
-        GMS_BATCH_SWITCH(BatchKernels<KK>::occupancy, (post), log_b, kv)                         \
+    int batch_occupancy_k##KK(int log_b, bool kv, bool post, uint32_t keys) {                \
+        GMS_BATCH_SWITCH(BatchKernels<KK>::occupancy, (post, keys), log_b, kv)                   \
         return 1;                                                                        \
     }
 
