@@ -987,6 +987,8 @@ class Batch:
 
     @property
     def tuning(self):
+        """The shape and grid in effect (of an untuned batch, the first step's shape);
+        setting items_per_thread 0 gives every step a shape by its size."""
         t = gms_batch_tuning()
         _check(lib().gms_batch_get_tuning(self._h, ctypes.byref(t)), "gms_batch_get_tuning")
         return {"items_per_thread": t.items_per_thread, "persistent": t.persistent}

@@ -688,8 +688,8 @@ gms_status gms_batch_launch_graph(gms_batch* b, void* stream) {
 
 gms_status gms_batch_set_tuning(gms_batch* b, gms_batch_tuning t) {
     if (!b) return GMS_ERR_INVALID_ARG;
-    if (t.items_per_thread != 8 && t.items_per_thread != 16 && t.items_per_thread != 24 &&
-        t.items_per_thread != 32)
+    if (t.items_per_thread != 0 && t.items_per_thread != 8 && t.items_per_thread != 16 &&
+        t.items_per_thread != 24 && t.items_per_thread != 32)
         return GMS_ERR_INVALID_ARG;
     if (t.persistent > 1) return GMS_ERR_INVALID_ARG;
     b->tuning.items_per_thread = t.items_per_thread;

@@ -427,9 +427,12 @@ typedef struct gms_batch_item {
     uint32_t *d_offsets;
 } gms_batch_item;
 
-/* Tile shape and grid of the batched kernels (picked by gms_batch_autotune). */
+/* Tile shape and grid of the batched kernels.  A batch that was not tuned (or
+ * was set to 0) takes, for each of its steps, a shape by the step's keys and
+ * bucket counts; gms_batch_autotune and gms_batch_set_tuning give all steps one. */
 typedef struct gms_batch_tuning {
-    uint32_t items_per_thread;  /* 8, 16, 24 or 32: tile = 256 x items_per_thread keys */
+    uint32_t items_per_thread;  /* 8, 16, 24 or 32: tile = 256 x items_per_thread keys;
+                                   set to 0: by size, step by step */
     uint32_t persistent;        /* 0: one workgroup per tile; 1: resident grid
                                    pulling tiles from a device work queue */
 } gms_batch_tuning;
@@ -511,10 +514,14 @@ gms_status gms_batch_launch_graph(gms_batch *b, void *stream);
 gms_status gms_batch_autotune(gms_batch *b, uint32_t reps, void *stream,
                               gms_batch_tuning *chosen, float *ms_per_run);
 gms_status gms_batch_set_tuning(gms_batch *b, gms_batch_tuning t);
+/* The tuning in effect; of a batch whose shapes go by size, that of the first
+ * step (24 before the first plan).  Writing it back fixes that shape for every
+ * step: set 0 to return to shapes by size. */
 gms_status gms_batch_get_tuning(const gms_batch *b, gms_batch_tuning *t);
 
 /* Shape of the current plan: keys, work items (tiles), matrix words, kernel
- * launches per run. */
+ * launches per run at most (a step's scan counts as three; it takes one up to
+ * 2^23 matrix words). */
 gms_status gms_batch_stats(const gms_batch *b, uint64_t *keys, uint32_t *work_items,
                            uint64_t *matrix_words, uint32_t *launches);
 

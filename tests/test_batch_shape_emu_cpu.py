@@ -41,3 +41,34 @@ def _shape(emu, parts):  # noqa: F811
     ([(1_000_000, 32, 0)] * 35 + [(1_000_000, 64, 0)] * 37, 24)])
 def test_default_shape(emu, parts, items):  # noqa: F811
     assert _shape(emu, parts) == items
+
+
+def test_by_size_can_be_restored(emu):  # noqa: F811
+    """Reading the tuning and writing it back fixes the first step's shape for every
+    step; 0 returns to shapes by size."""
+    items = [gms.gms_batch_item((1 << 40) + (i << 34), None, (2 << 40) + (i << 34), None, 1_000_000, 64,
+                                gms.range_bucket(64).desc(), None) for i in range(42)]
+    arr = (gms.gms_batch_item * len(items))(*items)
+    sort = gms.gms_batch_sort_item(3 << 40, None, 4 << 40, None, 5000, 8)
+    h, t = ctypes.c_void_p(), gms.gms_batch_tuning()
+    work = ctypes.c_uint32()
+
+    def tiles():
+        assert emu.gms_batch_stats(h, None, ctypes.byref(work), None, None) == 0
+        return work.value
+
+    assert emu.gms_batch_create(ctypes.byref(h)) == 0
+    try:
+        assert emu.gms_batch_plan_mixed(h, arr, len(items), ctypes.byref(sort), 1, None) == 0
+        assert emu.gms_batch_get_tuning(h, ctypes.byref(t)) == 0
+        assert t.items_per_thread == 16
+        # step 0: the multisplits and the first digit, 16 keys per thread; three more digits, 8
+        first = 42 * -(-1_000_000 // 4096) + 2
+        assert tiles() == first + 3 * 3
+        assert emu.gms_batch_set_tuning(h, t) == 0
+        assert tiles() == first + 3 * 2
+        assert emu.gms_batch_set_tuning(h, gms.gms_batch_tuning(0, 0)) == 0
+        assert tiles() == first + 3 * 3
+        assert emu.gms_batch_set_tuning(h, gms.gms_batch_tuning(12, 0)) == 1
+    finally:
+        emu.gms_batch_destroy(h)
