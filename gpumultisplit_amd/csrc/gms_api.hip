@@ -1,5 +1,6 @@
 // C-ABI entry points (include/gpumultisplit.h) and the host-side engine.
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -374,7 +375,11 @@ static gms_status run_stages(Scratch& s, const uint32_t* kin, const uint32_t* vi
     MsCall c;
     gms_status st = plan_call(s, kin, vin, kout, vout, n, B, kv, stream, c);
     if (st != GMS_SUCCESS) return st;
-    c.reg_rank = reg_rank(c.log_b, kv, n, d_offsets && apart, pass);
+    // the postscans of the longer tiles of large inputs have no register form
+    const bool has_reg = reg_rank_starts_below(c.log_b, kv) != 0 &&
+                         !(c.large && tune_items(c.log_b, kv, true) != tune_items(c.log_b, kv, false));
+    c.reg_rank = has_reg &&
+                 form(Form::reg_postscan, reg_rank(c.log_b, kv, n, d_offsets && apart, pass));
     if (c.reg_rank && apart) {
         c.offs = d_offsets;
         c.nb = B;
@@ -1321,7 +1326,19 @@ gms_status gms_copy_u32(const uint32_t* src, uint32_t* dst, size_t n, void* stre
 }  // extern "C"
 
 #ifdef GMS_HOST_EMULATION
-// Test hook of the CPU emulation build only: the postscan's form.
+// Test hooks of the CPU emulation build only.  GMS_EMU_FORMS, four digits of 0, 1 or
+// '-' in the order of Form, forces forms from the start; gms_emu_force one later.
+namespace gms {
+int emu_forced[4] = {-1, -1, -1, -1};
+static const bool emu_forms_read = [] {
+    const char* v = getenv("GMS_EMU_FORMS");
+    for (int i = 0; v && i < 4 && v[i]; ++i)
+        if (v[i] == '0' || v[i] == '1') emu_forced[i] = v[i] - '0';
+    return true;
+}();
+}  // namespace gms
+extern "C" void gms_emu_force(int form, int value) { gms::emu_forced[form] = value; }
+// The postscan's form.
 extern "C" int gms_emu_reg_rank(int log_b, int kv, uint32_t n, int starts, int pass) {
     return gms::reg_rank(log_b, kv != 0, n, starts != 0, pass != 0);
 }

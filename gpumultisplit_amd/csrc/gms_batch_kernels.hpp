@@ -399,7 +399,7 @@ struct BatchKernels {
             return fn(std::true_type{});
         } else {
             if constexpr (from != kNoLds)
-                if (keys >= from) return fn(std::true_type{});
+                if (form(Form::batch_lds, keys >= from)) return fn(std::true_type{});
             return fn(std::false_type{});
         }
     }

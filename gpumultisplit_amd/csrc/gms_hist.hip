@@ -383,7 +383,7 @@ static hipError_t launch_range(const void* x, uint32_t n, int32_t* d_hist, uint3
     const uint32_t* xb = reinterpret_cast<const uint32_t*>(x);
     uint32_t* h = reinterpret_cast<uint32_t*>(d_hist);
     const dim3 grid(hist_grid(n, kRangeGrid)), block(kThreads);
-    if (n / kHistTile < kRangeGrid)
+    if (!form(Form::range_table, n / kHistTile >= kRangeGrid))
         hipLaunchKernelGGL((hist_range_kernel<T, false, false>), grid, block, 0, stream, xb, n,
                            num_levels, d_levels, h);
     else if (!stream_words(n))

@@ -123,7 +123,8 @@ hipError_t two_shape(const ShortCall& c, const ShortPlan& p, uint32_t* H, const 
 // 32-bit ids would take four times two launches instead), and 6144 where four
 // words per element leave no LDS for more.
 bool short_one_block(uint32_t n, uint32_t bits, uint32_t kw, uint32_t vw) {
-    return n <= (bits > 8u && bits <= 12u ? 4096u : kw + vw > 3u ? 6144u : 8192u);
+    return n <= (bits > 8u && bits <= 12u ? 4096u : kw + vw > 3u ? 6144u : 8192u) &&
+           form(Form::short_calls, true);
 }
 
 // Tiles of 4 elements per thread while that gives at most one tile per CU, then
@@ -169,7 +170,8 @@ ShortPlan short_plan(uint32_t n, uint32_t num_buckets, uint32_t kw, uint32_t vw)
     const int cl = ceil_log2_u32(num_buckets);
     const uint32_t lb = cl < 2 ? 2u : (uint32_t)cl;
     const bool wide = kw == 2 || vw == 2;
-    if (lb > (wide ? 8u : 10u) || n > short_top(lb, wide) || (!wide && whole_tiles_win(n, lb)))
+    if (lb > (wide ? 8u : 10u) || n > short_top(lb, wide) || (!wide && whole_tiles_win(n, lb)) ||
+        !form(Form::short_calls, true))
         return ShortPlan{0u, 1u, lb, 0u};
     return short_shape(n, lb);
 }

@@ -69,6 +69,20 @@ constexpr bool tune_alias(int log_b, int items, bool kv, int level_bits) {
     return kv && cnt_row(1 << level_bits) <= items && !(log_b >= 7 && items < 28);
 }
 
+// Choices between forms of the same results.  The tests of the CPU emulation build
+// force them (gms_emu_force; short_calls only off), as its sizes stay below most limits;
+// the GPU library always goes by the rule.
+enum class Form { short_calls, reg_postscan, range_table, batch_lds };
+#ifdef GMS_HOST_EMULATION
+extern int emu_forced[4];  // per Form: -1 by the rule, 0 or 1
+inline bool form(Form f, bool rule) {
+    const int v = emu_forced[(int)f];
+    return v < 0 ? rule : v != 0;
+}
+#else
+constexpr bool form(Form, bool rule) { return rule; }
+#endif
+
 // Few buckets: the classes whose postscan loads its tile through LDS and ranks it with
 // register counters (ms_postscan_reg_kernel), instead of blocked loads and LDS
 // counters, whenever the call wants the bucket starts, and from some size on without.
