@@ -21,7 +21,10 @@ namespace {
 // fiber runs until it meets a wave or workgroup barrier; the scheduler in
 // launch() lets it go on when every live fiber of its wave (workgroup) waits
 // at one.  (One host thread per GPU thread spent nearly all its time in
-// futex calls.)
+// futex calls.)  Fibers run one after another, so a missing barrier shows only
+// when the reader runs before the writer: every other workgroup runs its waves
+// and lanes in descending order, and the next launch the others.  A race that
+// needs two fibers between the same barriers to interleave does not show.
 enum class State { ready, at_wave, at_block, done };
 constexpr size_t kStack = 96 * 1024;
 struct Fiber {
@@ -153,7 +156,11 @@ void launch(dim3 grid, dim3 block, std::function<void()> body) {
         g_fibers.back()->stack.reset(new char[kStack]);
     }
     g_body = &body;
+    static uint32_t launches = 0;
+    ++launches;
+    const uint32_t waves = (nt + 63) / 64;
     for (uint32_t b = 0; b < grid.x; ++b) {
+        const bool down = ((b + launches) & 1u) != 0;
         block_idx = {b, 0, 0};
         for (uint32_t t = 0; t < nt; ++t) {
             Fiber& f = *g_fibers[t];
@@ -166,11 +173,13 @@ void launch(dim3 grid, dim3 block, std::function<void()> body) {
         }
         for (bool live = true; live;) {
             live = false;
-            for (uint32_t w = 0; w < nt; w += 64) {  // every wave up to its workgroup barrier
+            for (uint32_t v = 0; v < waves; ++v) {  // every wave up to its workgroup barrier
+                const uint32_t w = (down ? waves - 1 - v : v) * 64;
                 const uint32_t end = w + 64 < nt ? w + 64 : nt;
                 for (bool again = true; again;) {
                     uint32_t at_wave = 0, at_block = 0;
-                    for (uint32_t t = w; t < end; ++t) {
+                    for (uint32_t i = w; i < end; ++i) {
+                        const uint32_t t = down ? w + end - 1 - i : i;
                         if (g_fibers[t]->state == State::ready) run_fiber(t);
                         at_wave += g_fibers[t]->state == State::at_wave;
                         at_block += g_fibers[t]->state == State::at_block;

@@ -4,7 +4,8 @@
 // tests of the real kernel code at small sizes).
 //
 // Execution model: a kernel launch runs its workgroups one after another;
-// every workgroup is blockDim.x fibers that meet at __syncthreads().
+// every workgroup is blockDim.x fibers that meet at __syncthreads(), run in
+// ascending order in one workgroup and in descending order in the next.
 // __shared__ arrays become function-static storage, which
 // is what LDS is to a sequence of workgroups.  DPP lane moves and readlane
 // are wave collectives: the 64 threads of a wave publish their values and
