@@ -218,7 +218,10 @@ uint32_t gms_tile_keys(uint32_t num_buckets, int key_value, uint32_t n);
 /* Stage timing for measurement: when enabled, every multisplit on this context
  * records HIP events on its stream around the prescan, scan and postscan
  * kernels.  gms_multisplit_profile synchronises and returns the summed
- * milliseconds and the number of recorded calls since the last reset. */
+ * milliseconds and the number of recorded calls since the last reset.  Short
+ * calls have fewer kernels (gpumultisplit_amd/csrc/gms_short.hpp): of two
+ * launches the count is the prescan and the scatter, which scans too, the
+ * postscan; a call of one launch counts as postscan, the other two as zero. */
 gms_status gms_multisplit_set_profiling(gms_multisplit_ctx *ctx, int enable);
 gms_status gms_multisplit_profile(gms_multisplit_ctx *ctx, double *ms_prescan,
                                   double *ms_scan, double *ms_postscan,
