@@ -42,14 +42,16 @@ void large_scratch_free(LargeScratch& L) {
     L.cap = 0;
 }
 
-// Passes of equal width where no key distribution measured slower, else 8 bits
-// a pass.  On MI355X, time over that of 8 bits a pass, uniform / sorted / nine in ten
-// keys equal:
-//   12 bits  6 + 6: 1.6M .91 / .83 / .84; 9M key-only .99 / 1.07 / 1.07, key-value .94 /
-//            1.05 / 1.03; 2^25 key-value .96 / 1.01 / 1.00, 50M .94 / .95 / .98
+// Passes of equal width where that measured faster, or on no key distribution more
+// than a few percent slower than it is faster on others; else 8 bits a pass.  On
+// MI355X, on buffers that change from call to call, time over that of 8 bits a
+// pass, uniform / sorted / nine in ten keys equal:
+//   12 bits  6 + 6: 2M .87 / .79 / .79, 2.2M 1.03 / 1.06 / 1.05, 2.6M .99 / 1.06 / 1.02; key-value 3M
+//            .94 / 1.03 / 1.01, 4M .91 / 1.00 / .98, 9M .95 / 1.02 / 1.02, 2^25 .96 / .99 / 1.00;
+//            key-only 3.5M 1.04 / 1.12 / 1.11, 9M .98 / 1.05 / 1.04
 //   13 bits  7 + 6: 1.1M .96 / .96 / .96, 3M .91 / .97 / .97, 2^24 .98 / 1.00 / 1.00
-//   14 bits  7 + 7: 1.9M 1.18 / 1.26 / 1.23, 2^27 key-only 1.08 / 1.07 / 1.04, key-value .95 /
-//            1.10 / 1.04
+//   14 bits  7 + 7: 2M 1.15 / 1.21 / 1.18, 3M .93 / .95 / .94, 9M key-only .97 / .98 / .98, key-value
+//            .98 / 1.00 / .99; 2^27 key-only 1.08 / 1.07 / 1.04, key-value .95 / 1.10 / 1.04
 //   17 bits  9 + 8: 1M .85 / .85 / .88, 9M .84 / .85 / .85, 2^27 key-value .77 / .81 / .81,
 //            key-only .88 / 1.10 / 1.00 but 6 + 6 + 5 .95 / 1.00 / .97
 //   18 bits  9 + 9: 1M .91 / .91 / .99, 9M .91 / .94 / .93, 2^27 key-value .83 / .90 / .91,
@@ -63,8 +65,9 @@ int large_passes(uint32_t bits, bool kv, bool wide, uint32_t n, uint32_t (&width
     bool even = false;
     if (!wide) {
         switch (bits) {
-            case 12: even = n <= 1u << 21 || (kv && n >= 1u << 25); break;
+            case 12: even = n <= 1u << 21 || (kv && n >= 11u << 18); break;
             case 13: even = true; break;
+            case 14: even = n > 1u << 21 && n < 1u << 26; break;
             case 17:
             case 18:
                 even = !(bits == 18 && n > 1u << 20 && n <= 3u << 19);

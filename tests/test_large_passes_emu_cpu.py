@@ -35,10 +35,11 @@ def test_no_width_that_measured_slower(emu):  # noqa: F811
     assert _passes(emu, 18, 1, 1 << 27) == [9, 9] and _passes(emu, 18, 0, 1 << 25) == [9, 9]
     assert _passes(emu, 18, 1, 1_300_000) == [8, 8, 2] and _passes(emu, 18, 1, 1 << 20) == [9, 9]
     for kv in (0, 1):
-        for n in SIZES:
+        for n in (1, 1 << 21, 1 << 26, 1 << 27):
             assert _passes(emu, 14, kv, n) == [8, 6]
-    assert _passes(emu, 12, 0, 9_000_000) == [8, 4] == _passes(emu, 12, 1, 9_000_000)
-    assert _passes(emu, 12, 1, 1 << 25) == [6, 6] == _passes(emu, 12, 0, 1 << 21)
+        assert _passes(emu, 14, kv, 3_000_000) == [7, 7]
+    assert _passes(emu, 12, 0, 9_000_000) == [8, 4] == _passes(emu, 12, 1, 2_600_000)
+    assert _passes(emu, 12, 1, 3_000_000) == [6, 6] == _passes(emu, 12, 0, 1 << 21)
     assert _passes(emu, 19, 1, 3_000_000) == [8, 8, 3] and _passes(emu, 20, 1, 1_900_000) == [8, 8, 4]
 
 
