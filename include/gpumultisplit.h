@@ -136,7 +136,9 @@ gms_status gms_multisplit_key_value(gms_multisplit_ctx *ctx, const uint32_t *d_k
 
 /* Same as the two above (d_value_in/out NULL = key-only) but writes the B
  * bucket starts to device memory d_offsets without blocking.  Replaces the
- * reference's B-1 blocking 4-byte copies (src/api/multisplit.cuh:144-149). */
+ * reference's B-1 blocking 4-byte copies (src/api/multisplit.cuh:144-149).  d_offsets may
+ * share memory with the call's inputs, which are read before the starts are
+ * written. */
 gms_status gms_multisplit(gms_multisplit_ctx *ctx, const uint32_t *d_key_in,
                           const uint32_t *d_value_in, uint32_t *d_key_out,
                           uint32_t *d_value_out, uint32_t n, gms_bucket_desc desc,
